@@ -575,6 +575,49 @@ __global__ __launch_bounds__(kAttnThreads) void attn_fwd_long_kernel(AttnArgs a)
     }
 }
 
+// A query tile of the long backward in flight: its Q, dO and O rows in staging
+// layout and, in the first lane of each row, the row's softmax statistics.
+template <int D>
+struct QueryTile {
+    f32x4 q[stage_units<D>()], dout[stage_units<D>()], o[stage_units<D>()];
+    f32x2 st[stage_units<D>()];
+};
+
+template <int D>
+__device__ __forceinline__ void query_tile_load(QueryTile<D>& t, const AttnArgs& a, int64_t base,
+                                                int item, int qt) {
+    tile_load<D>(t.q, a.q + base, a.ld, a.S, qt);
+    tile_load<D>(t.dout, a.dout + base, a.ld, a.S, qt);
+    tile_load<D>(t.o, a.o + base, a.ld, a.S, qt);
+    const int r0 = qt * kAttnSeq, rows = min(kAttnSeq, a.S - r0);
+    const auto rs = buffer_rsrc(a.stats + ((int64_t)item * a.S + r0) * 2, (int64_t)rows * 8);
+#pragma unroll
+    for (int u = 0; u < stage_units<D>(); ++u) {
+        const int row = (threadIdx.x + kAttnThreads * u) / (D / 4);
+        t.st[u] = buffer_load2(rs, row * 8);
+    }
+}
+
+// Stages the tile, and per query (max, 1/sum, dO . O): the row term is formed
+// from the staging registers, D/4 neighbouring lanes to a row.
+template <int D>
+__device__ __forceinline__ void query_tile_store(const QueryTile<D>& t, float* q_lds, float* do_lds,
+                                                 f32x4* st_lds) {
+#pragma unroll
+    for (int u = 0; u < stage_units<D>(); ++u) {
+        stage_store<D>(t.q, u, q_lds);
+        stage_store<D>(t.dout, u, do_lds);
+        float dot = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dot = fmaf(t.o[u][e], t.dout[u][e], dot);
+#pragma unroll
+        for (int m = 1; m < D / 4; m *= 2) dot += __shfl_xor(dot, m, 64);
+        const int idx = threadIdx.x + kAttnThreads * u;
+        if (idx % (D / 4) == 0)
+            st_lds[idx / (D / 4)] = f32x4{t.st[u][0], 1.0f / t.st[u][1], dot, 0.0f};
+    }
+}
+
 template <int D>
 __global__ __launch_bounds__(kAttnThreads) void attn_bwd_long_kernel(AttnArgs a) {
     constexpr int KP = D + 4, NJ = D / 16, U = stage_units<D>();
@@ -586,7 +629,6 @@ __global__ __launch_bounds__(kAttnThreads) void attn_bwd_long_kernel(AttnArgs a)
     __shared__ f32x4 st_lds[kAttnSeq];           // per query: max, 1/sum, dO . O
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int tid = threadIdx.x;
     const int S = a.S, T = (S + kAttnSeq - 1) / kAttnSeq;
     const int item = blockIdx.x / T, kt = blockIdx.x - item * T;
     const int64_t base = item_base(a, item, D);
@@ -615,38 +657,13 @@ __global__ __launch_bounds__(kAttnThreads) void attn_bwd_long_kernel(AttnArgs a)
         o_v[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         o_k[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
+    QueryTile<D> next;
+    query_tile_load<D>(next, a, base, item, 0);
     for (int qt = 0; qt < T; ++qt) {
         const int q0 = qt * kAttnSeq;
-        {
-            f32x4 qv[U], dv[U];
-            tile_load<D>(qv, a.q + base, a.ld, S, qt);
-            tile_load<D>(dv, a.dout + base, a.ld, S, qt);
-            f32x4 stv = f32x4{0.0f, 1.0f, 0.0f, 0.0f};
-            if (tid < kAttnSeq && q0 + tid < S) {
-                const int64_t row = q0 + tid;
-                const float* st = a.stats + ((int64_t)item * S + row) * 2;
-                // the softmax backward's row term: dO . O of this query
-                float dot = 0.0f;
-                const auto ro = buffer_rsrc(a.o + base + row * a.ld, D * 4);
-                const auto rd = buffer_rsrc(a.dout + base + row * a.ld, D * 4);
-                float ov[D], dd[D];
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    ov[d] = buffer_load1(ro, 4 * d);
-                    dd[d] = buffer_load1(rd, 4 * d);
-                }
-#pragma unroll
-                for (int d = 0; d < D; ++d) dot = fmaf(ov[d], dd[d], dot);
-                stv = f32x4{st[0], 1.0f / st[1], dot, 0.0f};
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                stage_store<D>(qv, u, q_lds);
-                stage_store<D>(dv, u, do_lds);
-            }
-            if (tid < kAttnSeq) st_lds[tid] = stv;
-        }
+        query_tile_store<D>(next, q_lds, do_lds, st_lds);
         __syncthreads();
+        if (qt + 1 < T) query_tile_load<D>(next, a, base, item, qt + 1);
         // lane (c, g): key krow, queries qb*16 + 4g + r of the tile
         f32x4 p[8], dp[8];
         scores_t<D, 0, 8>(p, q_lds, kf, c, g);
@@ -688,7 +705,8 @@ __global__ __launch_bounds__(kAttnThreads) void attn_bwd_long_kernel(AttnArgs a)
                 const int ql = 16 * w + 4 * g + r;
                 if (q0 + ql < S) part[(int64_t)ql * D + j * 16 + c] = o_q[j][r];
             }
-        __syncthreads();  // q_lds, do_lds, x_lds and st_lds are restaged next
+        // q_lds, do_lds and st_lds, restaged next, were last read before the
+        // barrier above; x_lds is written again only after the next one
     }
     // dK, dV of this workgroup's keys (rows k0 + 16w + 4g + r)
     f32x4 old_k[NJ], old_v[NJ];
