@@ -317,6 +317,101 @@ void launch_splitk_reduce(GemmArgs p, int slices) { launch_reduce(p, slices); }
 
 namespace {
 
+// Sums split-K partials and applies the epilogue. A workgroup covers 64
+// consecutive outputs with kSplitGroups slice groups: group y sums slices
+// [y*per, (y+1)*per) in ascending order, then the group sums are added in
+// group order. The order depends only on the slice count, so the result is
+// deterministic; every partial read is a coalesced 64-float row segment.
+constexpr int kSplitGroups = 16;
+
+__global__ __launch_bounds__(64 * kSplitGroups) void splitk_reduce_kernel(GemmArgs p,
+                                                                         int slices) {
+    __shared__ float red[kSplitGroups][64];
+    const int64_t total = p.mrows * p.N;
+    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+    const int per = (slices + kSplitGroups - 1) / kSplitGroups;
+    const int s0 = min(slices, ty * per), s1 = min(slices, s0 + per);
+    for (int64_t base = (int64_t)blockIdx.x * 64; base < total; base += (int64_t)gridDim.x * 64) {
+        const int64_t e = base + tx;
+        float v = 0.0f;
+        if (e < total)
+            for (int s = s0; s < s1; ++s) v += p.partial[(int64_t)s * total + e];
+        red[ty][tx] = v;
+        __syncthreads();
+        if (ty == 0 && e < total) {
+            float r = red[0][tx];
+#pragma unroll
+            for (int y = 1; y < kSplitGroups; ++y) r += red[y][tx];
+            const int64_t row = e / p.N;
+            if (row < p.M) {
+                epilogue_store(p, p.C, row, e - row * p.N, r);
+            } else {  // the row of sums
+                float* sr = p.sum_row + (e - row * p.N);
+                if (p.sum_beta != 0.0f) r = r + p.sum_beta * *sr;
+                *sr = r;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// The same sum for row-major outputs of whole float4s (N % 4 == 0, C and the
+// partials 16-byte aligned): a thread owns four consecutive outputs and adds
+// the slices in slice order with 128-bit loads, eight (then four) slices'
+// loads in flight at a time; no LDS, no barrier. Row-major epilogue only.
+__global__ __launch_bounds__(256) void splitk_reduce4_kernel(GemmArgs p, int slices) {
+    const int64_t total = p.mrows * p.N, total4 = total >> 2;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total4;
+         i += (int64_t)gridDim.x * 256) {
+        const f32x4* src = reinterpret_cast<const f32x4*>(p.partial) + i;
+        const int64_t stride4 = total4;
+        f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        int s = 0;
+        for (; s + 8 <= slices; s += 8) {
+            f32x4 v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = src[(int64_t)(s + j) * stride4];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc = acc + v[j];
+        }
+        if (s + 4 <= slices) {
+            f32x4 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = src[(int64_t)(s + j) * stride4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc = acc + v[j];
+            s += 4;
+        }
+        for (; s < slices; ++s) acc = acc + src[(int64_t)s * stride4];
+        const int64_t e = i << 2, row = e / p.N, col = e - row * p.N;
+        if (row < p.M) {
+            if (p.epi & NRS_EPI_BIAS_COL)
+                acc = acc + f32x4{p.bias[col], p.bias[col + 1], p.bias[col + 2], p.bias[col + 3]};
+            if (p.epi & NRS_EPI_BIAS_ROW) acc = acc + p.bias[row];
+            if (p.epi & NRS_EPI_RELU) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[j] = fmaxf(acc[j], 0.0f);
+            }
+            if (p.mask) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (!(p.mask[row * p.ldc + col + j] > 0.0f)) acc[j] = 0.0f;
+            }
+            f32x4* dst = reinterpret_cast<f32x4*>(p.C + row * p.ldc + col);
+            if (p.beta != 0.0f) acc = acc + p.beta * *dst;
+            *dst = acc;
+        } else {  // the row of sums
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float r = acc[j];
+                float* sr = p.sum_row + col + j;
+                if (p.sum_beta != 0.0f) r = r + p.sum_beta * *sr;
+                *sr = r;
+            }
+        }
+    }
+}
+
 void launch_reduce(GemmArgs p, int slices) {
     const int64_t total = p.mrows * p.N;
     if (p.N % 4 == 0 && p.nchw_P == 0 && p.ldc == p.N && aligned16(p.C) && aligned16(p.partial)) {
@@ -328,6 +423,98 @@ void launch_reduce(GemmArgs p, int slices) {
     unsigned blocks = (unsigned)std::min<int64_t>(cdiv(total, 64), 4 * (int64_t)num_cus());
     hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(64 * kSplitGroups), 0, stream(), p,
                        slices);
+}
+
+}  // namespace
+
+namespace {
+
+// Tiles of the split GEMM with what a k step of 32 costs a workgroup (us:
+// `alone` on its CU, `shared` with others there) and what it costs besides
+// (filling the pipeline, the epilogue), fitted to whole grids of
+// 1024^2, 2048^2 and 4096^2 over K = 32 .. 512, e.g. (us)
+//   4096^2 over 64 / 512   256x256 24 / 90    128x128 32 / 117   64x128 28 / 134
+//   2048^2 over 64 / 512   128x128 10 / 31    64x128 8.9 / 32    64x64 10 / 35
+//   1024^2 over 64 / 512   64x64K 5.1 / 11.3  64x64 5.2 / 13.6   128x128 7.5 / 21
+// (a 256x128 tile with second accumulators takes 660 us for 4096^3, the
+// 256x256 one 590).
+struct SplitShape {
+    int bm, bn, bk, threads;
+    double alone, shared, fixed;
+};
+const SplitShape kSplitShapes[S_COUNT] = {
+    {256, 256, 16, 512, 4.55, 4.55, 12.5},
+    {128, 128, 32, 512, 1.5, 1.5, 4.5},
+    {64, 128, 32, 256, 0.93, 0.9, 1.6},
+    {64, 64, 64, 512, 0.45, 0.5, 1.9},
+    {64, 64, 32, 256, 0.61, 0.456, 1.25},
+};
+
+// The split GEMM takes dense products of more than 32 rows and columns whose
+// rows leave a 32-bit offset over a tile (a row of ones is built for TN). The
+// f32 tiles keep gathered operands, outputs of at most 32 rows or columns
+// (padding would leave the matrix cores nothing to gain) and short
+// reductions, where a launch is all latency.
+bool split_eligible(const GemmCall& c) {
+    const int64_t lda = c.layout == NRS_TN ? c.M : c.K, ldb = c.layout == NRS_NT ? c.K : c.N;
+    return c.amode == OP_DENSE && c.bmode == OP_DENSE && c.M > 32 && c.N > 32 && c.K >= 32 &&
+           lda < (1 << 21) && ldb < (1 << 21) && (!c.sum_row || c.layout == NRS_TN) &&
+           c.force_slices <= 0;
+}
+
+// The group kernel takes any dense product the split GEMM's addressing and
+// row of ones allow.
+bool groupable(const GemmCall& c) {
+    const int64_t lda = c.layout == NRS_TN ? c.M : c.K, ldb = c.layout == NRS_NT ? c.K : c.N;
+    return c.amode == OP_DENSE && c.bmode == OP_DENSE && c.batch == 1 && c.nchw_P == 0 &&
+           c.partial_buf == nullptr && c.force_slices == 0 && c.K > 0 && lda < (1 << 21) &&
+           ldb < (1 << 21) && (!c.sum_row || c.layout == NRS_TN);
+}
+
+// The tile of the least estimated time. Outputs of few 64x64 tiles over a
+// long reduction are split over K as plan_gemm splits them.
+Plan plan_split(const GemmCall& c) {
+    const int64_t M = c.M + (c.sum_row ? 1 : 0), N = c.N, K = c.K;
+    const int64_t cus = num_cus();
+    const int64_t t64 = cdiv(M, 64) * cdiv(N, 64) * c.batch;
+    if (c.allow_split && c.nchw_P == 0 && c.batch == 1 && t64 < cus &&
+        (2 * t64 <= cus || K >= 2048) && K >= 256) {
+        const int64_t want = std::min<int64_t>(256, cdiv(3 * cus, t64));
+        const int64_t max_by_k = std::max<int64_t>(1, K / ((t64 >= 16 ? 8 : 2) * 32));
+        const int64_t slices = std::max<int64_t>(1, std::min(want, max_by_k));
+        const int64_t kps = cdiv(cdiv(K, slices), 32) * 32;
+        return Plan{S64x64, (int)cdiv(K, kps), kps, 0};
+    }
+    Plan best{S64x64, 1, K, 0};
+    double least = 1e30;
+    for (int t = 0; t < S_COUNT; ++t) {
+        const SplitShape& s = kSplitShapes[t];
+        const int64_t wgs = cdiv(M, s.bm) * cdiv(N, s.bn) * c.batch, per_cu = cdiv(wgs, cus);
+        const double steps = (double)(cdiv(K, s.bk) * s.bk) / 32.0;
+        const double step = per_cu > 1 ? s.shared : s.alone;
+        const double est = (double)per_cu * (steps * step + s.fixed);
+        if (est < least) {
+            least = est;
+            best.tile = t;
+        }
+    }
+    best.k_per_slice = cdiv(K, kSplitShapes[best.tile].bk) * kSplitShapes[best.tile].bk;
+    return best;
+}
+
+// Partials of a split-K launch: the caller's buffer or the library's scratch.
+int partials_for(const GemmCall& c, const Plan& pl, int64_t mrows, float*& ws) {
+    const size_t need = sizeof(float) * (size_t)pl.slices * (size_t)mrows * (size_t)c.N;
+    if (c.partial_buf) {
+        NRS_ARG_CHECK(need <= c.partial_cap,
+                      "gemm: split-K partials of %zu bytes (%d slices of %lld x %lld) exceed "
+                      "the %zu-byte scratch of the no-allocation entry point",
+                      need, pl.slices, (long long)c.M, (long long)c.N, c.partial_cap);
+        ws = c.partial_buf;
+        return NRS_OK;
+    }
+    ws = workspace(need, 0);
+    return ws ? NRS_OK : NRS_ERR_ALLOC;
 }
 
 }  // namespace
@@ -345,41 +532,37 @@ int gemm_run(const GemmCall& c) {
     if (skinny_eligible(c)) return skinny_run(c);
     const bool dense = c.amode == OP_DENSE && c.bmode == OP_DENSE;
     const bool vec4 = vec4_loads(c);
+    const bool split = split_eligible(c);
 
-    Plan pl = plan_gemm(M + (c.sum_row ? 1 : 0), N, K, batch, vec4, dense,
-                        c.allow_split && c.nchw_P == 0, c.force_slices);
-    const TileShape& s = kShapes[pl.tile];
+    const Plan pl = split ? plan_split(c)
+                          : plan_gemm(M + (c.sum_row ? 1 : 0), N, K, batch, vec4, dense,
+                                      c.allow_split && c.nchw_P == 0, c.force_slices);
+    TileShape s;
+    KernelFn fn;
+    if (split) {
+        const SplitShape& ss = kSplitShapes[pl.tile];
+        s = TileShape{ss.bm, ss.bn, ss.bk, ss.threads};
+        fn = split_kernel(pl.tile, layout);
+    } else {
+        s = kShapes[pl.tile];
+        fn = kernel_for(pl.tile, pl.pf, layout, vec4, c.amode, c.bmode);
+    }
+    NRS_ARG_CHECK(fn != nullptr, "gemm: no kernel for layout %d with operand modes %d/%d", layout,
+                  c.amode, c.bmode);
     GemmArgs p;
     const int arc = make_args(p, c, s, pl);
     if (arc != NRS_OK) return arc;
-
-    KernelFn fn = kernel_for(pl.tile, pl.pf, layout, vec4, c.amode, c.bmode);
-    NRS_ARG_CHECK(fn != nullptr, "gemm: no kernel for layout %d with operand modes %d/%d", layout,
-                  c.amode, c.bmode);
     dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)pl.slices, (unsigned)batch);
     if (pl.slices > 1) {
         NRS_ARG_CHECK(batch == 1, "gemm: split-K with batch > 1 unsupported");
-        const size_t need = sizeof(float) * (size_t)pl.slices * (size_t)p.mrows * (size_t)N;
-        float* ws;
-        if (c.partial_buf) {
-            NRS_ARG_CHECK(need <= c.partial_cap,
-                          "gemm: split-K partials of %zu bytes (%d slices of %lld x %lld) exceed "
-                          "the %zu-byte scratch of the no-allocation entry point",
-                          need, pl.slices, (long long)M, (long long)N, c.partial_cap);
-            ws = c.partial_buf;
-        } else {
-            ws = workspace(need, 0);
-            if (!ws) return NRS_ERR_ALLOC;
-        }
-        p.partial = ws;
-        hipLaunchKernelGGL(fn, grid, dim3(s.threads), 0, stream(), p);
-        NRS_LAUNCH_CHECK("gemm (split-K partials)");
+        const int wrc = partials_for(c, pl, p.mrows, p.partial);
+        if (wrc != NRS_OK) return wrc;
+    }
+    hipLaunchKernelGGL(fn, grid, dim3(s.threads), 0, stream(), p);
+    NRS_LAUNCH_CHECK(pl.slices > 1 ? "gemm (split-K partials)" : "gemm");
+    if (pl.slices > 1) {
         launch_reduce(p, pl.slices);
         NRS_LAUNCH_CHECK("gemm (split-K reduce)");
-    } else {
-        p.partial = nullptr;
-        hipLaunchKernelGGL(fn, grid, dim3(s.threads), 0, stream(), p);
-        NRS_LAUNCH_CHECK("gemm");
     }
     return NRS_OK;
 }
@@ -431,9 +614,7 @@ bool outputs_independent(const GemmCall* calls, int count, const OperandRange* e
 
 namespace {
 
-// The group kernel's tile: 64x64x32, 2x2 waves of 32x32, prefetch depth 2,
-// compiled for up to four waves per SIMD so that several problems'
-// workgroups share a CU.
+// The group kernel's tile.
 constexpr int kGroupBM = 64, kGroupBN = 64, kGroupBK = 32, kGroupThreads = 256;
 static_assert(kGroupMax >= NRS_GEMM_GROUP_MAX, "group size of the kernel and the C ABI");
 static_assert(sizeof(GemmGroupArgs) <= 4096, "group kernel arguments");
@@ -522,8 +703,7 @@ int launch_group(const GemmCall* calls, const GroupPlan& gp, float* partials, Ge
     if (part_of_call)
         for (int i = 0; i < kGroupMax; ++i) part_of_call[i] = part_of[i];
     NRS_ARG_CHECK(total_wgs <= INT32_MAX, "gemm group: grid too large");
-    hipLaunchKernelGGL((gemm_group_kernel<kGroupBM, kGroupBN, kGroupBK, 2, 2, 4, 2>),
-                       dim3((unsigned)total_wgs), dim3(kGroupThreads), 0, stream(), g);
+    hipLaunchKernelGGL(split_group_kernel(), dim3((unsigned)total_wgs), dim3(kGroupThreads), 0, stream(), g);
     NRS_LAUNCH_CHECK("gemm group");
     return NRS_OK;
 }
@@ -545,9 +725,7 @@ int gemm_group_run(const GemmCall* calls, int count) {
         ++live;
         if (i < kGroupMax) is_live[i] = true;
         const GemmCall& c = calls[i];
-        grouped = grouped && c.amode == OP_DENSE && c.bmode == OP_DENSE && c.batch == 1 &&
-                  c.nchw_P == 0 && c.partial_buf == nullptr && c.force_slices == 0 &&
-                  c.K > 0 && vec4_loads(c);
+        grouped = grouped && groupable(c);
         short_group = short_group && wsplit_eligible(c, true);
     }
     // An output overlapping another call's operand, bias or output would make

@@ -37,6 +37,27 @@ struct GemmArgs {
 
 
 
+// Tiles of the split GEMM (gemm_split.hpp), and its kernel for a tile and a
+// layout.
+enum SplitTile { S256x256 = 0, S128x128, S64x128, S64x64K, S64x64, S_COUNT };
+using SplitKernel = void (*)(GemmArgs);
+SplitKernel split_kernel(int tile, int layout);
+
+// Problems of one group launch: the C ABI's groups (NRS_GEMM_GROUP_MAX) and
+// the backward of three products sharing their left operand (three input-
+// gradient and three weight-gradient products).
+constexpr int kGroupMax = 6;
+struct GemmGroupArgs {
+    GemmArgs prob[kGroupMax];
+    int first[kGroupMax];   // first workgroup id of each problem, ascending
+    int layout[kGroupMax];  // NRS_NN / NRS_NT / NRS_TN
+    int slices[kGroupMax];  // K slices (partials to prob[q].partial when > 1)
+    int count;
+};
+// The group kernel: 64x64x32 tiles, 256 threads (gemm_split.hpp).
+using SplitGroupKernel = void (*)(GemmGroupArgs);
+SplitGroupKernel split_group_kernel();
+
 // Sums `slices` split-K partial tiles of p (p.partial, [slices][mrows][N]) in
 // slice order and applies p's epilogue (defined with the GEMM host code).
 void launch_splitk_reduce(GemmArgs p, int slices);

@@ -295,6 +295,151 @@ __device__ __forceinline__ void load_nchw(float (&r)[LOADS][VEC], __amdgpu_buffe
     }
 }
 
+// Where a lane's accumulators go: accumulator (i, j) element r is C[row, col]
+// with row = 32i + 8(r/4) + 4h + r%4, col = 32j + lane%32 inside the wave
+// tile. Every output column gets one base offset and a row stride, so element
+// (row, col) lands at base + row * stride: row-major C has base = col and
+// stride = ldc; NCHW C has base = img*M*P + (col - img*P) and stride = P;
+// split-K partials are row-major [M][N] per slice. The options (bias,
+// ReLU, beta) and the bounds tests are uniform per workgroup and hoisted
+// out of the element loop.
+template <int FN>
+struct TileOut {
+    float* out;
+    int64_t stride;
+    int64_t row0;  // row of element r = 0 of fragment i = 0
+    int64_t cbase[FN];
+    bool colok[FN];
+    bool full, plain;
+    float beta;
+};
+
+template <int BM, int BN, int FN>
+__device__ __forceinline__ TileOut<FN> tile_out(const GemmArgs& p, int64_t m0, int64_t n0, int wm0,
+                                                int wn0, int h, int l32, int slice,
+                                                int64_t batch) {
+    TileOut<FN> t;
+    t.full = (m0 + BM <= p.M) && (n0 + BN <= p.N);
+    t.plain =
+        p.partial != nullptr || (p.epi == NRS_EPI_NONE && p.beta == 0.0f && p.mask == nullptr);
+    if (p.partial) {
+        t.out = p.partial + (int64_t)slice * p.mrows * p.N;
+        t.stride = p.N;
+    } else {
+        t.out = p.C + batch * p.sC;
+        t.stride = p.nchw_P > 0 ? p.nchw_P : p.ldc;
+    }
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+        const int64_t col = n0 + wn0 + 32 * j + l32;
+        t.colok[j] = col < p.N;
+        if (p.partial == nullptr && p.nchw_P > 0) {
+            uint32_t img, pc;  // N < 2^31 (checked on the host)
+            fast_divmod((uint32_t)col, p.div_nchw, img, pc);
+            t.cbase[j] = (int64_t)img * p.M * p.nchw_P + pc;
+        } else {
+            t.cbase[j] = col;
+        }
+    }
+    t.row0 = m0 + wm0 + 4 * h;
+    t.beta = p.partial ? 0.0f : p.beta;
+    return t;
+}
+
+// The epilogue: bias, ReLU, mask, beta * old and the row of sums. `col0` is
+// the lane's column of fragment j = 0; with EARLY, the old values are passed
+// in (else they are loaded here).
+template <int FM, int FN, bool EARLY>
+__device__ __forceinline__ void tile_store(const GemmArgs& p, const TileOut<FN>& t,
+                                           const f32x16 (&acc)[FM][FN],
+                                           const float (&early)[EARLY ? FM : 1][EARLY ? FN : 1][16],
+                                           int64_t col0) {
+    float* const out = t.out;
+    const int64_t stride = t.stride, row0 = t.row0;
+    const float beta = t.beta;
+    if (t.plain && t.full) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                float* dst = out + t.cbase[j] + (row0 + 32 * i) * stride;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) dst[(8 * (r >> 2) + (r & 3)) * stride] = acc[i][j][r];
+            }
+    } else {
+        const bool bias_col = !p.partial && (p.epi & NRS_EPI_BIAS_COL);
+        const bool bias_row = !p.partial && (p.epi & NRS_EPI_BIAS_ROW);
+        const bool relu = !p.partial && (p.epi & NRS_EPI_RELU);
+        const float* mask = p.partial ? nullptr : p.mask;  // row-major C only
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            const float bc = (bias_col && t.colok[j]) ? p.bias[col0 + 32 * j] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+                // The fragment's 16 old values and row biases are loaded
+                // before any store, unconditionally from a clamped (always
+                // valid) address: a load inside the store's bounds branch
+                // would be sunk there by the compiler and cost a round trip
+                // per element. Values of lanes that store nothing are unused.
+                float old[16], br[16];
+                bool live[16];
+                if (beta != 0.0f || bias_row || mask) {  // uniform
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int64_t row = row0 + 32 * i + 8 * (r >> 2) + (r & 3);
+                        const bool ok = t.colok[j] & (row < p.M);
+                        if constexpr (EARLY)
+                            old[r] = beta != 0.0f ? early[i][j][r] : 0.0f;
+                        else
+                            old[r] = beta != 0.0f ? out[ok ? t.cbase[j] + row * stride : 0] : 0.0f;
+                        br[r] = bias_row ? p.bias[ok ? row : 0] : 0.0f;
+                        live[r] = mask ? mask[ok ? t.cbase[j] + row * stride : 0] > 0.0f : true;
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                // All 16 results first, each in a register of its own
+                // (pinned by the empty asm; they overwrite the old values):
+                // computed inside each store's bounds branch they would share
+                // one temporary, and a store's data register cannot be
+                // overwritten before the store has read it, so every store
+                // would wait for the one before it.
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float v = acc[i][j][r];
+                    if (bias_col) v += bc;
+                    if (bias_row) v += br[r];
+                    if (relu) v = fmaxf(v, 0.0f);
+                    if (mask && !live[r]) v = 0.0f;
+                    if (beta != 0.0f) v = v + beta * old[r];
+                    old[r] = v;
+                    asm volatile("" : "+v"(old[r]));
+                }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int64_t row = row0 + 32 * i + 8 * (r >> 2) + (r & 3);
+                    if (t.colok[j] && row < p.M) out[t.cbase[j] + row * stride] = old[r];
+                }
+                if (p.sum_row) {  // uniform; the row of sums, raw
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int64_t row = row0 + 32 * i + 8 * (r >> 2) + (r & 3);
+                        if (t.colok[j] && row == p.M) {
+                            if (p.partial) {
+                                out[t.cbase[j] + row * stride] = acc[i][j][r];
+                            } else {
+                                float* sr = p.sum_row + t.cbase[j];
+                                float v = acc[i][j][r];
+                                if (p.sum_beta != 0.0f) v = v + p.sum_beta * *sr;
+                                *sr = v;
+                            }
+                        }
+                    }
+                }
+            }
+        }
+    }
+}
+
 // Template parameters of gemm_block / gemm_kernel:
 // WPE (kernels): minimum waves per SIMD the register allocation must allow.
 // PF: prefetch depth. Global loads for k-tile j go into register slot j % PF
@@ -482,42 +627,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_
         }
     }
 
-    // Accumulator (i, j) element r of this lane is C[row, col] with
-    // row = 32i + 8(r/4) + 4h + r%4, col = 32j + lane%32 inside the wave tile.
-    // Every output column gets one base offset and a row stride, so element
-    // (row, col) lands at base + row * stride: row-major C has base = col and
-    // stride = ldc; NCHW C has base = img*M*P + (col - img*P) and stride = P;
-    // split-K partials are row-major [M][N] per slice. The options (bias,
-    // ReLU, beta) and the bounds tests are uniform per workgroup and hoisted
-    // out of the element loop.
-    const bool full = (m0 + BM <= p.M) && (n0 + BN <= p.N);
-    const bool plain =
-        p.partial != nullptr || (p.epi == NRS_EPI_NONE && p.beta == 0.0f && p.mask == nullptr);
-    float* out;
-    int64_t stride;
-    if (p.partial) {
-        out = p.partial + (int64_t)slice * p.mrows * p.N;
-        stride = p.N;
-    } else {
-        out = p.C + batch * p.sC;
-        stride = p.nchw_P > 0 ? p.nchw_P : p.ldc;
-    }
-    int64_t cbase[FN];
-    bool colok[FN];
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-        const int64_t col = n0 + wn0 + 32 * j + l32;
-        colok[j] = col < p.N;
-        if (p.partial == nullptr && p.nchw_P > 0) {
-            uint32_t img, pc;  // N < 2^31 (checked on the host)
-            fast_divmod((uint32_t)col, p.div_nchw, img, pc);
-            cbase[j] = (int64_t)img * p.M * p.nchw_P + pc;
-        } else {
-            cbase[j] = col;
-        }
-    }
-    const int64_t row0 = m0 + wm0 + 4 * h;  // row of element r = 0 of fragment i = 0
-    const float beta = p.partial ? 0.0f : p.beta;
+    const TileOut<FN> to = tile_out<BM, BN, FN>(p, m0, n0, wm0, wn0, h, l32, slice, batch);
     // Small wave tiles load the values an accumulating epilogue adds to
     // before the last k-tiles are reduced, so that round trip overlaps the
     // MFMAs instead of following them (clamped, always-valid addresses;
@@ -525,16 +635,16 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_
     constexpr bool kEarlyOld = FM * FN <= 2;
     float early[kEarlyOld ? FM : 1][kEarlyOld ? FN : 1][16];
     if constexpr (kEarlyOld) {
-        if (beta != 0.0f && kset == 0) {  // uniform
+        if (to.beta != 0.0f && kset == 0) {  // uniform
 #pragma unroll
             for (int i = 0; i < FM; ++i)
 #pragma unroll
                 for (int j = 0; j < FN; ++j)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        const int64_t row = row0 + 32 * i + 8 * (r >> 2) + (r & 3);
-                        const bool ok = colok[j] & (row < p.M);
-                        early[i][j][r] = out[ok ? cbase[j] + row * stride : 0];
+                        const int64_t row = to.row0 + 32 * i + 8 * (r >> 2) + (r & 3);
+                        const bool ok = to.colok[j] & (row < p.M);
+                        early[i][j][r] = to.out[ok ? to.cbase[j] + row * to.stride : 0];
                     }
         }
     }
@@ -584,87 +694,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_
                         acc[i][j][r] += smem[(((s2 * WS + wv) * FM + i) * FN + j) * 1024 + r * 64 + lane];
     }
 
-    if (plain && full) {
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                float* dst = out + cbase[j] + (row0 + 32 * i) * stride;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) dst[(8 * (r >> 2) + (r & 3)) * stride] = acc[i][j][r];
-            }
-    } else {
-        const bool bias_col = !p.partial && (p.epi & NRS_EPI_BIAS_COL);
-        const bool bias_row = !p.partial && (p.epi & NRS_EPI_BIAS_ROW);
-        const bool relu = !p.partial && (p.epi & NRS_EPI_RELU);
-        const float* mask = p.partial ? nullptr : p.mask;  // row-major C only
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            const float bc = (bias_col && colok[j]) ? p.bias[n0 + wn0 + 32 * j + l32] : 0.0f;
-#pragma unroll
-            for (int i = 0; i < FM; ++i) {
-                // The fragment's 16 old values and row biases are loaded
-                // before any store, unconditionally from a clamped (always
-                // valid) address: a load inside the store's bounds branch
-                // would be sunk there by the compiler and cost a round trip
-                // per element. Values of lanes that store nothing are unused.
-                float old[16], br[16];
-                bool live[16];
-                if (beta != 0.0f || bias_row || mask) {  // uniform
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int64_t row = row0 + 32 * i + 8 * (r >> 2) + (r & 3);
-                        const bool ok = colok[j] & (row < p.M);
-                        if constexpr (kEarlyOld)
-                            old[r] = beta != 0.0f ? early[i][j][r] : 0.0f;
-                        else
-                            old[r] = beta != 0.0f ? out[ok ? cbase[j] + row * stride : 0] : 0.0f;
-                        br[r] = bias_row ? p.bias[ok ? row : 0] : 0.0f;
-                        live[r] = mask ? mask[ok ? cbase[j] + row * stride : 0] > 0.0f : true;
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                // All 16 results first, each in a register of its own
-                // (pinned by the empty asm; they overwrite the old values):
-                // computed inside each store's bounds branch they would share
-                // one temporary, and a store's data register cannot be
-                // overwritten before the store has read it, so every store
-                // would wait for the one before it.
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    float v = acc[i][j][r];
-                    if (bias_col) v += bc;
-                    if (bias_row) v += br[r];
-                    if (relu) v = fmaxf(v, 0.0f);
-                    if (mask && !live[r]) v = 0.0f;
-                    if (beta != 0.0f) v = v + beta * old[r];
-                    old[r] = v;
-                    asm volatile("" : "+v"(old[r]));
-                }
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int64_t row = row0 + 32 * i + 8 * (r >> 2) + (r & 3);
-                    if (colok[j] && row < p.M) out[cbase[j] + row * stride] = old[r];
-                }
-                if (p.sum_row) {  // uniform; the row of sums, raw
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int64_t row = row0 + 32 * i + 8 * (r >> 2) + (r & 3);
-                        if (colok[j] && row == p.M) {
-                            if (p.partial) {
-                                out[cbase[j] + row * stride] = acc[i][j][r];
-                            } else {
-                                float* sr = p.sum_row + cbase[j];
-                                float v = acc[i][j][r];
-                                if (p.sum_beta != 0.0f) v = v + p.sum_beta * *sr;
-                                *sr = v;
-                            }
-                        }
-                    }
-                }
-            }
-        }
-    }
+    tile_store<FM, FN, kEarlyOld>(p, to, acc, early, n0 + wn0 + l32);
 }
 
 template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool AK, bool BKC, int VEC, int PF,
@@ -724,157 +754,6 @@ void gemm_kernel(GemmArgs p) {
         split_coords(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x, gridDim.y, bid, slice);
     gemm_block<BM, BN, BK, WAVES_M, WAVES_N, AK, BKC, VEC, PF, AMODE, BMODE, KS>(p, smem, bid, slice,
                                                                                  blockIdx.z);
-}
-
-// Several independent dense GEMMs in one launch (the products of one
-// backward step, or projections of one input): problem q owns workgroups
-// [first[q], first[q] + tiles_q * slices[q]) of a 1-D grid, each range
-// starting at a multiple of 8 so that a workgroup's XCD is its id within the
-// problem modulo 8, as in a launch of its own (ids past a problem's range,
-// the padding up to the next multiple of 8, exit at once). The problems'
-// workgroups share the CUs, so one problem's load latency, barriers and
-// epilogue overlap another's MFMAs; one launch per GEMM leaves each CU a
-// single workgroup of small tiles whose waves all stall at the same points.
-// Problems of one group launch: the C ABI's groups (NRS_GEMM_GROUP_MAX) and
-// the backward of three products sharing their left operand (three input-
-// gradient and three weight-gradient products).
-constexpr int kGroupMax = 6;
-struct GemmGroupArgs {
-    GemmArgs prob[kGroupMax];
-    int first[kGroupMax];   // first workgroup id of each problem, ascending
-    int layout[kGroupMax];  // NRS_NN / NRS_NT / NRS_TN
-    int slices[kGroupMax];  // K slices (partials to prob[q].partial when > 1)
-    int count;
-};
-
-template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int WPE, int PF>
-__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) __attribute__((amdgpu_waves_per_eu(WPE)))
-void gemm_group_kernel(GemmGroupArgs g) {
-    constexpr int kNN = 2 * Cfg<BM, BN, BK, WAVES_M, WAVES_N, true, false, 4>::STAGE;
-    constexpr int kNT = 2 * Cfg<BM, BN, BK, WAVES_M, WAVES_N, true, true, 4>::STAGE;
-    constexpr int kTN = 2 * Cfg<BM, BN, BK, WAVES_M, WAVES_N, false, false, 4>::STAGE;
-    constexpr int kMax = kNN > kNT ? (kNN > kTN ? kNN : kTN) : (kNT > kTN ? kNT : kTN);
-    __shared__ __attribute__((aligned(16))) float smem[kMax];
-    const int b = blockIdx.x;
-    int q = 0;
-#pragma unroll
-    for (int i = 1; i < kGroupMax; ++i)
-        if (i < g.count && b >= g.first[i]) q = i;
-    const GemmArgs& p = g.prob[q];
-    const int tiles = p.tiles_m * p.tiles_n, slices = g.slices[q];
-    const int lin = b - g.first[q];
-    if (lin >= tiles * slices) return;  // uniform: padding up to the next problem
-    int bid, slice;
-    split_coords(lin, tiles, slices, bid, slice);
-    switch (g.layout[q]) {
-        case NRS_NN:
-            gemm_block<BM, BN, BK, WAVES_M, WAVES_N, true, false, 4, PF, OP_DENSE, OP_DENSE, 1>(
-                p, smem, bid, slice, 0);
-            break;
-        case NRS_NT:
-            gemm_block<BM, BN, BK, WAVES_M, WAVES_N, true, true, 4, PF, OP_DENSE, OP_DENSE, 1>(
-                p, smem, bid, slice, 0);
-            break;
-        default:
-            gemm_block<BM, BN, BK, WAVES_M, WAVES_N, false, false, 4, PF, OP_DENSE, OP_DENSE, 1>(
-                p, smem, bid, slice, 0);
-            break;
-    }
-}
-
-// Sums split-K partials and applies the epilogue. A workgroup covers 64
-// consecutive outputs with kSplitGroups slice groups: group y sums slices
-// [y*per, (y+1)*per) in ascending order, then the group sums are added in
-// group order. The order depends only on the slice count, so the result is
-// deterministic; every partial read is a coalesced 64-float row segment.
-constexpr int kSplitGroups = 16;
-
-__global__ __launch_bounds__(64 * kSplitGroups) void splitk_reduce_kernel(GemmArgs p,
-                                                                         int slices) {
-    __shared__ float red[kSplitGroups][64];
-    const int64_t total = p.mrows * p.N;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int per = (slices + kSplitGroups - 1) / kSplitGroups;
-    const int s0 = min(slices, ty * per), s1 = min(slices, s0 + per);
-    for (int64_t base = (int64_t)blockIdx.x * 64; base < total; base += (int64_t)gridDim.x * 64) {
-        const int64_t e = base + tx;
-        float v = 0.0f;
-        if (e < total)
-            for (int s = s0; s < s1; ++s) v += p.partial[(int64_t)s * total + e];
-        red[ty][tx] = v;
-        __syncthreads();
-        if (ty == 0 && e < total) {
-            float r = red[0][tx];
-#pragma unroll
-            for (int y = 1; y < kSplitGroups; ++y) r += red[y][tx];
-            const int64_t row = e / p.N;
-            if (row < p.M) {
-                epilogue_store(p, p.C, row, e - row * p.N, r);
-            } else {  // the row of sums
-                float* sr = p.sum_row + (e - row * p.N);
-                if (p.sum_beta != 0.0f) r = r + p.sum_beta * *sr;
-                *sr = r;
-            }
-        }
-        __syncthreads();
-    }
-}
-
-// The same sum for row-major outputs of whole float4s (N % 4 == 0, C and the
-// partials 16-byte aligned): a thread owns four consecutive outputs and adds
-// the slices in slice order with 128-bit loads, eight (then four) slices'
-// loads in flight at a time; no LDS, no barrier. Row-major epilogue only.
-__global__ __launch_bounds__(256) void splitk_reduce4_kernel(GemmArgs p, int slices) {
-    const int64_t total = p.mrows * p.N, total4 = total >> 2;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total4;
-         i += (int64_t)gridDim.x * 256) {
-        const f32x4* src = reinterpret_cast<const f32x4*>(p.partial) + i;
-        const int64_t stride4 = total4;
-        f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        int s = 0;
-        for (; s + 8 <= slices; s += 8) {
-            f32x4 v[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = src[(int64_t)(s + j) * stride4];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc = acc + v[j];
-        }
-        if (s + 4 <= slices) {
-            f32x4 v[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = src[(int64_t)(s + j) * stride4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc = acc + v[j];
-            s += 4;
-        }
-        for (; s < slices; ++s) acc = acc + src[(int64_t)s * stride4];
-        const int64_t e = i << 2, row = e / p.N, col = e - row * p.N;
-        if (row < p.M) {
-            if (p.epi & NRS_EPI_BIAS_COL)
-                acc = acc + f32x4{p.bias[col], p.bias[col + 1], p.bias[col + 2], p.bias[col + 3]};
-            if (p.epi & NRS_EPI_BIAS_ROW) acc = acc + p.bias[row];
-            if (p.epi & NRS_EPI_RELU) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[j] = fmaxf(acc[j], 0.0f);
-            }
-            if (p.mask) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (!(p.mask[row * p.ldc + col + j] > 0.0f)) acc[j] = 0.0f;
-            }
-            f32x4* dst = reinterpret_cast<f32x4*>(p.C + row * p.ldc + col);
-            if (p.beta != 0.0f) acc = acc + p.beta * *dst;
-            *dst = acc;
-        } else {  // the row of sums
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                float r = acc[j];
-                float* sr = p.sum_row + col + j;
-                if (p.sum_beta != 0.0f) r = r + p.sum_beta * *sr;
-                *sr = r;
-            }
-        }
-    }
 }
 
 }  // namespace nrs

@@ -1,0 +1,182 @@
+"""The split GEMM (gemm_split.hpp): f32 products as six products of bf16 pieces.
+
+Shapes cover every tile of its planner at the places it can go wrong: whole
+tiles, one row or column past a tile, k remainders under and over a step,
+misaligned operands (odd leading dimensions, pointers off 16 bytes), K slices.
+
+Bars: bit-exact where every product and partial sum is an integer below 2^24
+(one operand of up to 18 bits, so all three of its pieces carry bits); against
+f64, |C - C64| <= (6 K / 16 + 8) * 2^-24 * (|A||B|) element by element: each
+instruction rounds once, six products a step of 16, and the three products of
+pieces left out are below 2^-25 of theirs.
+"""
+import numpy as np
+import pytest
+
+from kat import int_matrix
+
+pytestmark = pytest.mark.gpu
+
+NN, NT, TN = 0, 1, 2
+
+SHAPES = [  # rows, cols, inner
+    (33, 33, 32), (64, 64, 64), (65, 63, 33), (129, 200, 47),
+    (1000, 1333, 65),      # 64x64 or 64x128 tiles, ragged everywhere
+    (1500, 1500, 100), (2048, 2048, 96), (2049, 2047, 80),  # 128x128 tiles
+    (4096, 256, 130),      # k-split wave sets
+    (4100, 4090, 40), (4096, 4096, 48),  # 256x256 tiles
+    (64, 576, 5000), (70, 130, 4099), (520, 260, 2100),  # K slices
+]
+IDS = lambda s: "x".join(map(str, s))
+
+
+def operands(layout, rows, cols, inner, make_a, make_b):
+    a = make_a((rows, inner) if layout != TN else (inner, rows))
+    b = make_b((inner, cols) if layout != NT else (cols, inner))
+    return a, b
+
+
+def logical(layout, a, b):
+    return (a.T if layout == TN else a).astype(np.float64), \
+           (b.T if layout == NT else b).astype(np.float64)
+
+
+def upload(hip, x, offset):
+    """x on the device, `offset` floats past a 16-byte boundary."""
+    buf = hip.DeviceBuffer.from_host(np.concatenate([np.zeros(offset, np.float32), x.ravel()]))
+    return buf, buf.ptr + 4 * offset
+
+
+def gemm(hip, layout, a, b, rows, cols, inner, offset=0, **kw):
+    keep_a, pa = upload(hip, a, offset)
+    keep_b, pb = upload(hip, b, offset)
+    c = hip.DeviceBuffer.from_host(kw.pop("c0", np.full((rows, cols), np.nan, np.float32)))
+    hip.gemm(layout, c, pa, pb, rows, cols, inner, **kw)
+    return c.to_host((rows, cols))
+
+
+@pytest.mark.parametrize("layout", [NN, NT, TN])
+@pytest.mark.parametrize("shape", SHAPES, ids=IDS)
+def test_exact_integers_all_pieces(hip, layout, shape):
+    rows, cols, inner = shape
+    rng = np.random.default_rng(rows + 3 * cols + 7 * inner + layout)
+    bits = min(18, 23 - int(np.ceil(np.log2(inner))))  # sums of inner of them stay below 2^24
+    wide = lambda s: int_matrix(rng, s, -2 ** bits + 1, 2 ** bits - 1)
+    sign = lambda s: int_matrix(rng, s, -1, 1)
+    for offset, (ma, mb) in enumerate([(wide, sign), (sign, wide)]):
+        a, b = operands(layout, rows, cols, inner, ma, mb)
+        A, B = logical(layout, a, b)
+        got = gemm(hip, layout, a, b, rows, cols, inner, offset=offset)
+        assert np.array_equal(got.astype(np.float64), A @ B)
+
+
+@pytest.mark.parametrize("layout", [NN, NT, TN])
+@pytest.mark.parametrize("shape", [(33, 33, 32), (129, 200, 47), (1000, 1333, 777),
+                                   (2049, 2047, 300), (4096, 256, 1024), (64, 576, 20001)],
+                         ids=IDS)
+def test_f64_error(hip, layout, shape):
+    rows, cols, inner = shape
+    rng = np.random.default_rng(rows + cols + inner + layout)
+    # magnitudes over nine decades
+    make = lambda s: (rng.standard_normal(s) * 10.0 ** rng.integers(-6, 4, s)).astype(np.float32)
+    a, b = operands(layout, rows, cols, inner, make, make)
+    A, B = logical(layout, a, b)
+    sample = np.unique(np.linspace(0, rows - 1, 97).astype(int))
+    got = gemm(hip, layout, a, b, rows, cols, inner)[sample]
+    bound = (6 * inner / 16 + 8) * 2.0 ** -24 * (np.abs(A[sample]) @ np.abs(B))
+    assert np.all(np.abs(got - A[sample] @ B) <= bound)
+
+
+@pytest.mark.parametrize("layout", [NN, NT, TN])
+@pytest.mark.parametrize("shape", [(129, 200, 70), (1500, 1500, 100), (4096, 256, 130)], ids=IDS)
+def test_epilogues_exact(hip, layout, shape):
+    rows, cols, inner = shape
+    rng = np.random.default_rng(rows + layout)
+    small = lambda s: int_matrix(rng, s, -8, 8)
+    a, b = operands(layout, rows, cols, inner, small, small)
+    A, B = logical(layout, a, b)
+    c0, bc, br = small((rows, cols)), small(cols), small(rows)
+    got = gemm(hip, layout, a, b, rows, cols, inner, c0=c0, beta=2.0, bias=hip.DeviceBuffer.from_host(bc),
+               epilogue=hip.EPI_BIAS_COL | hip.EPI_RELU)
+    assert np.array_equal(got, np.maximum(A @ B + bc, 0) + 2 * c0)
+    got = gemm(hip, layout, a, b, rows, cols, inner, bias=hip.DeviceBuffer.from_host(br),
+               epilogue=hip.EPI_BIAS_ROW)
+    assert np.array_equal(got, A @ B + br[:, None])
+
+
+@pytest.mark.parametrize("layout", [NN, NT, TN])
+@pytest.mark.parametrize("shape", [(129, 200, 70), (1500, 1500, 100), (64, 576, 5000),
+                                   (4096, 256, 130), (4096, 4096, 48)], ids=IDS)
+def test_infinities_nan_and_overflow(hip, layout, shape):
+    """The results that are not finite are those of f32 multiplication and
+    addition, and every other result is untouched by them."""
+    rows, cols, inner = shape
+    rng = np.random.default_rng(7 * rows + layout)
+    small = lambda s: int_matrix(rng, s, 1, 8)  # no zeros: inf * 0 only where put
+    a, b = operands(layout, rows, cols, inner, small, small)
+    A, B = (a.T if layout == TN else a), (b.T if layout == NT else b)  # views
+    A[3, 5] = np.inf
+    A[rows - 1, inner - 1] = -np.inf
+    A[7, 2] = np.nan
+    B[4, cols - 2] = np.inf
+    B[5, 1] = 0.0                          # inf * 0
+    A[11, 0] = np.float32(3.4028235e38)    # rounds past bf16's range, finite
+    B[0, :] = 0.5
+    got = gemm(hip, layout, a, b, rows, cols, inner)
+    with np.errstate(all="ignore"):
+        want = np.zeros((rows, cols), np.float64)
+        fa, fb = np.where(np.isfinite(A), A, 0).astype(np.float64), \
+            np.where(np.isfinite(B), B, 0).astype(np.float64)
+        want = fa @ fb
+        for r, k in ((3, 5), (rows - 1, inner - 1), (7, 2)):
+            want[r] += np.float64(A[r, k]) * B[k].astype(np.float64)
+        want[:, cols - 2] += A[:, 4].astype(np.float64) * np.inf
+    big = np.zeros((rows, cols), bool)
+    big[11] = True
+    finite = np.isfinite(want) & ~big
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
+    assert np.array_equal(got[finite].astype(np.float64), want[finite])
+    row = np.isfinite(want[11])
+    assert np.allclose(got[11][row], want[11][row], rtol=2.0 ** -22)
+
+
+@pytest.mark.parametrize("layout", [NN, NT, TN])
+@pytest.mark.parametrize("shape", [(129, 200, 70), (1500, 1500, 100), (4096, 256, 130)], ids=IDS)
+def test_tiny_magnitudes(hip, layout, shape):
+    """Operands whose third piece lies under bf16's smallest denormal (2^-133)
+    lose no precision: the results are those of f32 products."""
+    rows, cols, inner = shape
+    rng = np.random.default_rng(5 * rows + layout)
+    tiny = lambda s: np.ldexp(rng.standard_normal(s), -118).astype(np.float32)
+    unit = lambda s: np.ldexp(rng.standard_normal(s), 20).astype(np.float32)
+    a, b = operands(layout, rows, cols, inner, tiny, unit)
+    A, B = logical(layout, a, b)
+    sample = np.unique(np.linspace(0, rows - 1, 97).astype(int))
+    got = gemm(hip, layout, a, b, rows, cols, inner)[sample]
+    bound = (inner + 8) * 2.0 ** -24 * (np.abs(A[sample]) @ np.abs(B))
+    assert np.all(np.abs(got - A[sample] @ B) <= bound)
+
+
+def test_bmm_large_items(hip):
+    """Batched items past the small-item kernel, each at its own offset."""
+    rng = np.random.default_rng(1)
+    batch, m, n, k = 5, 150, 131, 77
+    a, b = int_matrix(rng, (batch, m, k)), int_matrix(rng, (batch, k, n))
+    c = hip.DeviceBuffer(batch * m * n)
+    hip.bmm(NN, c, hip.DeviceBuffer.from_host(a), hip.DeviceBuffer.from_host(b), batch, m, n, k)
+    assert np.array_equal(c.to_host((batch, m, n)), a @ b)
+
+
+@pytest.mark.parametrize("batch,in_f", [(4096, 256), (500, 128), (300, 100)])
+def test_row_of_sums(hip, batch, in_f):
+    """A weight gradient alone, with its bias gradient as a row of sums (a tile
+    row of its own where in_f is a multiple of 64)."""
+    rng = np.random.default_rng(batch)
+    out_f = 192
+    x, g = int_matrix(rng, (batch, in_f), -2, 2), int_matrix(rng, (batch, out_f), -2, 2)
+    dw, db = hip.DeviceBuffer(in_f * out_f), hip.DeviceBuffer(out_f)
+    hip.call("nrs_linear_backward", None, dw, db, hip.DeviceBuffer.from_host(g),
+             hip.DeviceBuffer.from_host(x), None, batch, in_f, out_f, 0.0, 0.0, 0.0)
+    assert np.array_equal(dw.to_host((in_f, out_f)), x.T @ g)
+    assert np.array_equal(db.to_host(), g.sum(0))
