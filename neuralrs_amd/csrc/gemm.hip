@@ -57,40 +57,24 @@ KernelFn pick_conv(int layout, int amode, int bmode, bool vec4) {
     return nullptr;
 }
 
-// Tile configurations (chosen by a sweep over the workload shapes on MI355X).
-// All run two waves per SIMD (register budget capped at 256 per lane,
-// accumulators in VGPRs):
-//  * 256x256x32, 8 waves of 128x64, ~140 KB LDS, prefetch depth 1: large
-//    GEMMs (83-85% of FP32 MFMA peak at 4096^3 and 8192^3);
-//  * 64x64x32, 4 waves of 32x32, prefetch depth 2: everything mid-sized
-//    (bmm items, conv GEMMs, projections, split-K weight gradients);
-//  * 128x128x32, 8 waves of 64x32, prefetch depth 2: dense GEMMs with one
-//    to three of its tiles per CU (2048^3: 132 vs 150 us on 64x128; the cfg4
-//    FFN 4096x1024x256: 24.6 vs 24.9 us);
-//  * 64x128x32, 4 waves of 32x64, prefetch depth 2: grids of at least two
-//    of its tiles per CU and K >= 256 whose 128x128 grid would be mostly
-//    padding (2048^3 ran 162 us on it against 175 us on 64x64);
+// Tile configurations of the f32 kernels, for what the split GEMM does not
+// take (chosen by a sweep over the workload shapes on MI355X). All run two
+// waves per SIMD (register budget capped at 256 per lane, accumulators in
+// VGPRs):
+//  * 64x64x32, 4 waves of 32x32, prefetch depth 2: gathered (convolution)
+//    operands, and dense ones outside the other tiles and the split GEMM;
 //  * 32x256x32, 4 waves of 32x64, prefetch depth 2 (1 with scalar loads):
 //    outputs with at most 32 rows;
 //  * 32x128x32, 4 waves of 32x32, prefetch depth 2: convolutions whose GEMM
 //    has at most 32 rows (a 64-row tile would double the MFMA work);
 //  * 128x32x32, 4 waves of 32x32, prefetch depth 2: outputs with at most 32
-//    columns, e.g. attention's P.V and its input gradients (d_head 32);
-//  * 64x64x32 with k-split wave sets (KS = 2: 8 waves, two per 32x32
-//    sub-block, each reducing half of every k-tile), prefetch depth 2: dense
-//    GEMMs with at most two 64x64 tiles per CU and no K split, which would
-//    otherwise run one wave per SIMD (cfg4 projections 4096x256x256:
-//    9.3 -> 8.7 us NT; FFN 4096x256x1024: 29.0 -> 25.1 us NN).
-enum TileId { T256x256 = 0, T64x64, T32x256, T32x128, T128x32, T64x128, T64x64S2, T128x128, T_COUNT };
+//    columns, e.g. attention's P.V and its input gradients (d_head 32).
+enum TileId { T64x64 = 0, T32x256, T32x128, T128x32, T_COUNT };
 const TileShape kShapes[T_COUNT] = {
-    {256, 256, 32, 512},
     {64, 64, 32, 256},
     {32, 256, 32, 256},
     {32, 128, 32, 256},
     {128, 32, 32, 256},
-    {64, 128, 32, 256},
-    {64, 64, 32, 512},
-    {128, 128, 32, 512},
 };
 
 // `pf` is the register prefetch depth the plan asks for; tiles that have no
@@ -104,27 +88,15 @@ KernelFn kernel_for(int tile, int pf, int layout, bool vec4, int amode, int bmod
         }
     }
     switch (tile) {
-        case T256x256: return pick_layout<256, 256, 32, 2, 4, 1>(layout, vec4);
         case T64x64:
             return pf == 1 ? pick_layout<64, 64, 32, 2, 2, 1>(layout, vec4)
                            : pick_layout<64, 64, 32, 2, 2, 2>(layout, vec4);
         case T32x256:  // depth 2 with 128-bit loads; its scalar-load variant needs depth 1
             return vec4 ? pick_fixed<32, 256, 32, 1, 4, 2, 4>(layout)
                         : pick_fixed<32, 256, 32, 1, 4, 1, 1>(layout);
-        case T64x128:  // planned only with 128-bit loads (the scalar variant spills)
-            return vec4 ? pick_fixed<64, 128, 32, 2, 2, 2, 4>(layout) : nullptr;
         case T128x32:
             return pf == 1 ? pick_layout<128, 32, 32, 4, 1, 1>(layout, vec4)
                            : pick_layout<128, 32, 32, 4, 1, 2>(layout, vec4);
-        case T128x128:  // planned only with 128-bit loads
-            return vec4 ? pick_fixed<128, 128, 32, 2, 4, 2, 4>(layout) : nullptr;
-        case T64x64S2:  // planned only with 128-bit loads
-            if (!vec4) return nullptr;
-            switch (layout) {
-                case NRS_NN: return gemm_kernel<64, 64, 32, 2, 2, true, false, 4, 2, 2, OP_DENSE, OP_DENSE, 2>;
-                case NRS_NT: return gemm_kernel<64, 64, 32, 2, 2, true, true, 4, 2, 2, OP_DENSE, OP_DENSE, 2>;
-                default: return gemm_kernel<64, 64, 32, 2, 2, false, false, 4, 2, 2, OP_DENSE, OP_DENSE, 2>;
-            }
         default: return nullptr;
     }
 }
@@ -140,19 +112,12 @@ struct Plan {
     int pf;  // register prefetch depth (k-tiles in flight per thread)
 };
 
-// Chooses the tile shape and the number of K slices. The 256x256 tile is
-// used only with 128-bit loads (its scalar-load variant spills) and when at
-// least 85% of its tile grid is real output.
+// Chooses the f32 tile and the number of K slices.
 Plan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t batch, bool vec4, bool dense,
-               bool allow_split, int force_slices) {
+               bool allow_split) {
     const int cus = num_cus();
     auto tiles_of = [&](int t) {
         return cdiv(M, kShapes[t].bm) * cdiv(N, kShapes[t].bn) * batch;
-    };
-    // fraction of a tile grid's area that is real output (the rest is padding)
-    auto fill = [&](int t) {
-        return (double)(M * N) / ((double)cdiv(M, kShapes[t].bm) * kShapes[t].bm *
-                                  cdiv(N, kShapes[t].bn) * kShapes[t].bn);
     };
     Plan pl{T64x64, 1, K, 2};
     if (dense) {
@@ -160,21 +125,13 @@ Plan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t batch, bool vec4, bool d
             pl.tile = T32x256;
         else if (N <= 32 && M >= 128 && vec4)  // its scalar-load variants spill
             pl.tile = T128x32;
-        else if (vec4 && tiles_of(T256x256) >= cus && fill(T256x256) >= 0.85)
-            pl.tile = T256x256;
-        else if (vec4 && tiles_of(T128x128) >= cus && fill(T128x128) >= 0.85)
-            pl.tile = T128x128;
-        else if (vec4 && tiles_of(T64x128) >= 2 * cus && K >= 256 && fill(T64x128) >= 0.85)
-            pl.tile = T64x128;
     } else if (M <= 32) {  // gathered (convolution) operands: 64x64 or 32x128
         pl.tile = T32x128;
     }
     const TileShape& s = kShapes[pl.tile];
     const int64_t tiles = tiles_of(pl.tile);
     int slices = 1;
-    if (force_slices > 0) {
-        slices = force_slices;
-    } else if (allow_split && batch == 1 && tiles < cus && (2 * tiles <= cus || K >= 2048) &&
+    if (allow_split && batch == 1 && tiles < cus && (2 * tiles <= cus || K >= 2048) &&
                K >= 8 * s.bk) {
         // (a K of fewer than 8 k-tiles is not split: the reduce launch
         // costs more than the shorter k loop saves, e.g. 256x784 over
@@ -194,10 +151,6 @@ Plan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t batch, bool vec4, bool d
         slices = (int)std::min<int64_t>(want, max_by_k);
     }
     if (slices < 1) slices = 1;
-    // Unsplit dense 64x64 grids of at most two tiles per CU: k-split wave sets.
-    if (dense && vec4 && slices == 1 && force_slices <= 0 && pl.tile == T64x64 &&
-        tiles <= 2 * (int64_t)cus && cdiv(K, s.bk) >= 2)
-        pl.tile = T64x64S2;
     int64_t kps = cdiv(cdiv(K, slices), s.bk) * s.bk;
     if (kps <= 0) kps = s.bk;
     slices = (int)std::max<int64_t>(1, cdiv(K, kps));
@@ -453,13 +406,14 @@ const SplitShape kSplitShapes[S_COUNT] = {
 // The split GEMM takes dense products of more than 32 rows and columns whose
 // rows leave a 32-bit offset over a tile (a row of ones is built for TN). The
 // f32 tiles keep gathered operands, outputs of at most 32 rows or columns
-// (padding would leave the matrix cores nothing to gain) and short
-// reductions, where a launch is all latency.
+// (padding would leave the matrix cores nothing to gain) and reductions under
+// a k step into few tiles (1024 x 1024 over 16: 4.4 us against 4.7; with four
+// tiles a CU the split tiles win again, 4096 x 4096 over 16: 23 against 17).
 bool split_eligible(const GemmCall& c) {
     const int64_t lda = c.layout == NRS_TN ? c.M : c.K, ldb = c.layout == NRS_NT ? c.K : c.N;
-    return c.amode == OP_DENSE && c.bmode == OP_DENSE && c.M > 32 && c.N > 32 && c.K >= 32 &&
-           lda < (1 << 21) && ldb < (1 << 21) && (!c.sum_row || c.layout == NRS_TN) &&
-           c.force_slices <= 0;
+    return c.amode == OP_DENSE && c.bmode == OP_DENSE && c.M > 32 && c.N > 32 && c.K > 0 &&
+           (c.K >= 32 || cdiv(c.M, 64) * cdiv(c.N, 64) * c.batch >= 4 * (int64_t)num_cus()) &&
+           lda < (1 << 21) && ldb < (1 << 21) && (!c.sum_row || c.layout == NRS_TN);
 }
 
 // The group kernel takes any dense product the split GEMM's addressing and
@@ -467,7 +421,7 @@ bool split_eligible(const GemmCall& c) {
 bool groupable(const GemmCall& c) {
     const int64_t lda = c.layout == NRS_TN ? c.M : c.K, ldb = c.layout == NRS_NT ? c.K : c.N;
     return c.amode == OP_DENSE && c.bmode == OP_DENSE && c.batch == 1 && c.nchw_P == 0 &&
-           c.partial_buf == nullptr && c.force_slices == 0 && c.K > 0 && lda < (1 << 21) &&
+           c.partial_buf == nullptr && c.K > 0 && lda < (1 << 21) &&
            ldb < (1 << 21) && (!c.sum_row || c.layout == NRS_TN);
 }
 
@@ -536,7 +490,7 @@ int gemm_run(const GemmCall& c) {
 
     const Plan pl = split ? plan_split(c)
                           : plan_gemm(M + (c.sum_row ? 1 : 0), N, K, batch, vec4, dense,
-                                      c.allow_split && c.nchw_P == 0, c.force_slices);
+                                      c.allow_split && c.nchw_P == 0);
     TileShape s;
     KernelFn fn;
     if (split) {

@@ -42,7 +42,6 @@ struct GemmCall {
     int epi = NRS_EPI_NONE;
     int64_t nchw_P = 0;       // > 0: C is stored NCHW [img][M][nchw_P]
     bool allow_split = true;  // split-K allowed (batch == 1, row-major C only)
-    int force_slices = 0;
     int amode = OP_DENSE, bmode = OP_DENSE;
     ConvGeom cg{};
     int64_t gather_bytes = 0;  // bytes of the gathered (non-dense) operand's tensor

@@ -51,9 +51,9 @@ __device__ __forceinline__ void tile_coords(const GemmArgs& p, int bid, int& tm,
     tn = in_group / gsize;
 }
 
-template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool AK, bool BKC, int VEC, int KS = 1>
+template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool AK, bool BKC, int VEC>
 struct Cfg {
-    static constexpr int NT = 64 * WAVES_M * WAVES_N * KS;
+    static constexpr int NT = 64 * WAVES_M * WAVES_N;
     static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
     static constexpr int FM = WM / 32, FN = WN / 32;
     static constexpr int SA = AK ? (BK + 4) : (BM + 8);
@@ -65,10 +65,11 @@ struct Cfg {
     static constexpr int B_LOADS = BN * BK / (VEC * NT);
     static_assert(FM >= 1 && FN >= 1, "wave tile must be at least 32x32");
     static_assert(FM * 32 * WAVES_M == BM && FN * 32 * WAVES_N == BN, "wave grid");
-    static_assert(BK % (8 * KS) == 0, "BK must split into groups of 8 per k-split wave set");
+    static_assert(BK % 8 == 0, "BK must split into groups of 8");
     static_assert(A_LOADS >= 1 && B_LOADS >= 1, "tile too small for the thread count");
     static_assert(A_LOADS * VEC * NT == BM * BK && B_LOADS * VEC * NT == BN * BK, "load split");
     static_assert(2 * STAGE * 4 <= 160 * 1024, "LDS budget");
+    static_assert(FM * FN <= 2, "wave tiles of at most two accumulators");
 };
 
 // Position of load q of a k-tile of one operand (same mapping for the global
@@ -444,15 +445,10 @@ __device__ __forceinline__ void tile_store(const GemmArgs& p, const TileOut<FN>&
 // WPE (kernels): minimum waves per SIMD the register allocation must allow.
 // PF: prefetch depth. Global loads for k-tile j go into register slot j % PF
 // and are issued PF tiles before tile j is stored to LDS, so each load has
-// PF tiles of MFMA work to land in (small tiles need PF > 1 to cover HBM
-// latency; the 256x256 tile has enough work per k-tile with PF = 1).
+// PF tiles of MFMA work to land in (one k-tile of these small tiles does not
+// cover HBM latency).
 // AMODE / BMODE: OperandMode of A and B (OP_NCHW needs AK, OP_IM2COL needs
 // !BKC).
-// KS: wave sets splitting each k-tile. KS = 2 runs two waves per output
-// sub-block, each reducing half of every k-tile's groups of 8, and adds the
-// second set's accumulators to the first's through LDS at the end (fixed
-// order): twice the waves per SIMD for tiles that would leave one wave per
-// SIMD waiting on its barrier and LDS reads.
 // INTERIOR (gemm_tile): the whole output tile lies inside C and the K slice
 // is a whole number of k-tiles, so dense operands load and store without
 // per-element bounds selects.
@@ -461,12 +457,12 @@ __device__ __forceinline__ void tile_store(const GemmArgs& p, const TileOut<FN>&
 // of batch item `batch` (partials: slice `slice`), staging through `smem`
 // (2 * STAGE floats); gemm_block finds the tile of workgroup `bid` and picks
 // the interior or the bounds-checked form; gemm_kernel runs one GEMM per
-// launch, gemm_group_kernel several.
+// launch.
 template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool AK, bool BKC, int VEC, int PF,
-          int AMODE, int BMODE, int KS, bool INTERIOR>
+          int AMODE, int BMODE, bool INTERIOR>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_t m0, int64_t n0,
                                           int64_t kbeg, int64_t kend, int slice, int64_t batch) {
-    using C_ = Cfg<BM, BN, BK, WAVES_M, WAVES_N, AK, BKC, VEC, KS>;
+    using C_ = Cfg<BM, BN, BK, WAVES_M, WAVES_N, AK, BKC, VEC>;
     static_assert(AMODE != OP_IM2COL && BMODE != OP_NCHW, "unsupported operand mode");
     static_assert(AMODE != OP_NCHW || AK, "OP_NCHW is a reduction-contiguous operand");
     static_assert(BMODE != OP_IM2COL || !BKC, "OP_IM2COL is a k-major operand");
@@ -475,12 +471,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    const int kset = wave / (WAVES_M * WAVES_N);  // k-split wave set
-    const int wv = wave - kset * (WAVES_M * WAVES_N);
     const int h = lane >> 5;
     const int l32 = lane & 31;
-    const int wm0 = (wv / WAVES_N) * C_::WM;
-    const int wn0 = (wv % WAVES_N) * C_::WN;
+    const int wm0 = (wave / WAVES_N) * C_::WM;
+    const int wn0 = (wave % WAVES_N) * C_::WN;
 
     const float* A = p.A + batch * p.sA;
     const float* B = p.B + batch * p.sB;
@@ -512,21 +506,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_
     // t + 1 goes from its register slot to the other LDS buffer, tile
     // t + 1 + PF is loaded into the freed slot; loads past the end are
     // masked or skipped), so the compiler can count the loads in flight and
-    // wait only for the slot it stores, PF tiles after issuing it. With kPeel it runs
+    // wait only for the slot it stores, PF tiles after issuing it. It runs
     // while tile t + 1 is real and the last tiles go through the tail below,
     // which loads nothing, stores no padding tile and reduces no padding tile
     // (a single-tile GEMM would otherwise wait one more memory round trip for
     // a padding tile before its epilogue).
-    // Wave tiles of at most two accumulators peel the tail; the large tiles
-    // keep one straight-line loop over the k-tile count rounded up to PF
-    // (padding tiles load as zeros): with 128 accumulator registers the
-    // peeled tail costs them spills, and their k loops are long.
-    constexpr bool kPeel = FM * FN <= 2;
-    // Loads past the slice's end are skipped (not clamped) where no padding
-    // tile is reduced: with kPeel, or with one tile in flight.
-    constexpr bool kSkipPast = kPeel || PF == 1;
-    static_assert(!INTERIOR || (kSkipPast && AMODE == OP_DENSE && BMODE == OP_DENSE),
-                  "interior tiles skip the loads past the end");
+    static_assert(!INTERIOR || (AMODE == OP_DENSE && BMODE == OP_DENSE),
+                  "interior tiles are dense");
     auto loadA = [&](float (&r)[C_::A_LOADS][VEC], int64_t k0) {
         if constexpr (AMODE == OP_NCHW)
             load_nchw<BM, BK, VEC, C_::A_LOADS, NT>(r, gather, p.cg.div_P, m0, p.M, k0, kend, tid);
@@ -565,7 +551,6 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_
     };
 
     const int ntiles = kend > kbeg ? (int)((kend - kbeg + BK - 1) / BK) : 0;
-    const int nloop = kPeel ? ntiles : (ntiles + PF - 1) / PF * PF;
     if (ntiles > 0) {
         loadA(ra[0], kbeg);
         loadB(rb[0], kbeg);
@@ -573,7 +558,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_
         storeB(smem + C_::A_ELEMS, rb[0], kbeg);
 #pragma unroll
         for (int j = 1; j <= PF; ++j) {
-            if ((!kPeel && !kSkipPast) || j < ntiles) {  // uniform
+            if (j < ntiles) {  // uniform
                 const int64_t kj = kbeg + (int64_t)j * BK;
                 loadA(ra[j % PF], kj);
                 loadB(rb[j % PF], kj);
@@ -586,8 +571,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_
         const float* sA = smem + (t & 1) * C_::STAGE;
         const float* sB = sA + C_::A_ELEMS;
 #pragma unroll
-        for (int gg = 0; gg < BK / 8 / KS; ++gg) {
-            const int g = kset * (BK / 8 / KS) + gg;
+        for (int g = 0; g < BK / 8; ++g) {
             f32x4 af[FM], bf[FN];
 #pragma unroll
             for (int i = 0; i < FM; ++i)
@@ -608,7 +592,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_
 
     // The loop is unrolled by PF so every register-slot index is a constant.
     int t0 = 0;
-    for (; kPeel ? t0 + PF < ntiles : t0 < nloop; t0 += PF) {
+    for (; t0 + PF < ntiles; t0 += PF) {
 #pragma unroll
         for (int u = 0; u < PF; ++u) {
             const int t = t0 + u;
@@ -619,7 +603,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_
             storeA(dA, ra[slot], ks);
             storeB(dA + C_::A_ELEMS, rb[slot], ks);
             const int64_t kn = kbeg + (int64_t)(t + 1 + PF) * BK;
-            if (!kSkipPast || kn < kend) {  // uniform
+            if (kn < kend) {  // uniform
                 loadA(ra[slot], kn);
                 loadB(rb[slot], kn);
             }
@@ -628,32 +612,29 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_
     }
 
     const TileOut<FN> to = tile_out<BM, BN, FN>(p, m0, n0, wm0, wn0, h, l32, slice, batch);
-    // Small wave tiles load the values an accumulating epilogue adds to
-    // before the last k-tiles are reduced, so that round trip overlaps the
-    // MFMAs instead of following them (clamped, always-valid addresses;
-    // values of lanes that store nothing are unused).
-    constexpr bool kEarlyOld = FM * FN <= 2;
-    float early[kEarlyOld ? FM : 1][kEarlyOld ? FN : 1][16];
-    if constexpr (kEarlyOld) {
-        if (to.beta != 0.0f && kset == 0) {  // uniform
+    // The values an accumulating epilogue adds to are loaded before the last
+    // k-tiles are reduced, so that round trip overlaps the MFMAs instead of
+    // following them (clamped, always-valid addresses; values of lanes that
+    // store nothing are unused).
+    float early[FM][FN][16];
+    if (to.beta != 0.0f) {  // uniform
 #pragma unroll
-            for (int i = 0; i < FM; ++i)
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
-                for (int j = 0; j < FN; ++j)
+            for (int j = 0; j < FN; ++j)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int64_t row = to.row0 + 32 * i + 8 * (r >> 2) + (r & 3);
-                        const bool ok = to.colok[j] & (row < p.M);
-                        early[i][j][r] = to.out[ok ? to.cbase[j] + row * to.stride : 0];
-                    }
-        }
+                for (int r = 0; r < 16; ++r) {
+                    const int64_t row = to.row0 + 32 * i + 8 * (r >> 2) + (r & 3);
+                    const bool ok = to.colok[j] & (row < p.M);
+                    early[i][j][r] = to.out[ok ? to.cbase[j] + row * to.stride : 0];
+                }
     }
 
     // Tail: the last (at most PF) tiles; only real tiles are stored and reduced.
 #pragma unroll
     for (int u = 0; u < PF; ++u) {
         const int t = t0 + u;
-        if (kPeel && t < ntiles) {  // uniform
+        if (t < ntiles) {  // uniform
             reduce_tile(t);
             if (t + 1 < ntiles) {
                 const int slot = (u + 1) % PF;
@@ -666,57 +647,26 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, float* smem, int64_
         }
     }
 
-    if constexpr (KS > 1) {
-        // the other wave sets' accumulators, added to set 0's in set order
-        constexpr int WS = WAVES_M * WAVES_N;
-        static_assert((KS - 1) * WS * FM * FN * 16 * 64 <= 2 * C_::STAGE, "k-split LDS space");
-        __syncthreads();  // every wave is done with the staging buffers
-        if (kset > 0) {
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        smem[((((kset - 1) * WS + wv) * FM + i) * FN + j) * 1024 + r * 64 + lane] =
-                            acc[i][j][r];
-        }
-        __syncthreads();
-        if (kset > 0) return;  // uniform; no barrier follows
-#pragma unroll
-        for (int s2 = 0; s2 < KS - 1; ++s2)
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        acc[i][j][r] += smem[(((s2 * WS + wv) * FM + i) * FN + j) * 1024 + r * 64 + lane];
-    }
-
-    tile_store<FM, FN, kEarlyOld>(p, to, acc, early, n0 + wn0 + l32);
+    tile_store<FM, FN, true>(p, to, acc, early, n0 + wn0 + l32);
 }
 
 template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool AK, bool BKC, int VEC, int PF,
-          int AMODE, int BMODE, int KS>
+          int AMODE, int BMODE>
 __device__ __forceinline__ void gemm_block(const GemmArgs& p, float* smem, int bid, int slice,
                                            int64_t batch) {
-    using C_ = Cfg<BM, BN, BK, WAVES_M, WAVES_N, AK, BKC, VEC, KS>;
     int tm, tn;
     tile_coords(p, bid, tm, tn);
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
     const int64_t kbeg = (int64_t)slice * p.k_per_slice;
     const int64_t kend = min(p.K, kbeg + p.k_per_slice);
-    constexpr bool kInteriorForm =
-        AMODE == OP_DENSE && BMODE == OP_DENSE && (C_::FM * C_::FN <= 2 || PF == 1);
-    if constexpr (kInteriorForm) {
+    if constexpr (AMODE == OP_DENSE && BMODE == OP_DENSE) {
         if (m0 + BM <= p.M && n0 + BN <= p.N && (kend - kbeg) % BK == 0) {  // uniform
-            gemm_tile<BM, BN, BK, WAVES_M, WAVES_N, AK, BKC, VEC, PF, AMODE, BMODE, KS, true>(
+            gemm_tile<BM, BN, BK, WAVES_M, WAVES_N, AK, BKC, VEC, PF, AMODE, BMODE, true>(
                 p, smem, m0, n0, kbeg, kend, slice, batch);
             return;
         }
     }
-    gemm_tile<BM, BN, BK, WAVES_M, WAVES_N, AK, BKC, VEC, PF, AMODE, BMODE, KS, false>(
+    gemm_tile<BM, BN, BK, WAVES_M, WAVES_N, AK, BKC, VEC, PF, AMODE, BMODE, false>(
         p, smem, m0, n0, kbeg, kend, slice, batch);
 }
 
@@ -744,15 +694,15 @@ __device__ __forceinline__ void split_coords(int lin, int tiles, int slices, int
 }
 
 template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool AK, bool BKC, int VEC, int WPE,
-          int PF = 1, int AMODE = OP_DENSE, int BMODE = OP_DENSE, int KS = 1>
-__global__ __launch_bounds__(64 * WAVES_M * WAVES_N * KS) __attribute__((amdgpu_waves_per_eu(WPE)))
+          int PF = 1, int AMODE = OP_DENSE, int BMODE = OP_DENSE>
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) __attribute__((amdgpu_waves_per_eu(WPE)))
 void gemm_kernel(GemmArgs p) {
-    using C_ = Cfg<BM, BN, BK, WAVES_M, WAVES_N, AK, BKC, VEC, KS>;
+    using C_ = Cfg<BM, BN, BK, WAVES_M, WAVES_N, AK, BKC, VEC>;
     __shared__ __attribute__((aligned(16))) float smem[2 * C_::STAGE];
     int bid = blockIdx.x, slice = blockIdx.y;
     if (gridDim.y > 1 && (gridDim.x & 7) != 0)
         split_coords(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x, gridDim.y, bid, slice);
-    gemm_block<BM, BN, BK, WAVES_M, WAVES_N, AK, BKC, VEC, PF, AMODE, BMODE, KS>(p, smem, bid, slice,
+    gemm_block<BM, BN, BK, WAVES_M, WAVES_N, AK, BKC, VEC, PF, AMODE, BMODE>(p, smem, bid, slice,
                                                                                  blockIdx.z);
 }
 

@@ -134,7 +134,7 @@ bool aligned16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 
 bool skinny_eligible(const GemmCall& c) {
     if (c.amode != OP_DENSE || c.bmode != OP_DENSE || c.batch != 1 || c.nchw_P != 0 ||
-        c.force_slices != 0 || c.sum_row != nullptr || c.layout == NRS_NT)
+        c.sum_row != nullptr || c.layout == NRS_NT)
         return false;
     if (c.M < 1 || c.M > 32 || c.N < 1024 || c.K < 256 || c.N % 4 != 0 || !aligned16(c.B))
         return false;

@@ -274,7 +274,7 @@ bool wsplit_eligible(const GemmCall& c, bool automatic) {
     // (a caller-provided partials buffer does not matter: this kernel keeps
     // its partial sums on chip)
     if (c.amode != OP_DENSE || c.bmode != OP_DENSE || c.batch != 1 || c.nchw_P != 0 ||
-        c.force_slices != 0 || c.K < 1 || c.M < 1 || c.N < 1)
+        c.K < 1 || c.M < 1 || c.N < 1)
         return false;
     if (c.epi & ~(NRS_EPI_BIAS_COL | NRS_EPI_BIAS_ROW | NRS_EPI_RELU)) return false;
     if (c.K > kWsMaxK || c.M >= (1 << 30) || c.N >= (1 << 30)) return false;
