@@ -1271,10 +1271,57 @@ int small_wgrad(float* dweight, float* dbias, const float* grad, const float* in
     return wgrad_partial_sum(dweight, dbias, pw, pb, (int)d.N, (int)d.c_out, 1, (int)taps, beta);
 }
 
+// Whether the split tiles take a convolution ahead of the kernels that hold
+// their operands in LDS (split_conv may still refuse it). It is an estimate
+// against each, us on both sides, from sweeps over 8 .. 256 channels, 7x7 ..
+// 64x64 images and batches of 1 .. 256:
+// - small "same" 3x3 images, whose kernels give an image and a block of
+//   outputs to a workgroup, so they take whole rounds of the CUs whatever the
+//   image holds: N 64 128->128 14^2 36 against 45 (kept), 8^2 34 / 25, N 256
+//   256->256 8^2 492 / 112, N 8 64->64 14^2 20 / 16.5;
+// - the slab kernel is ahead by its one launch less where the reduction and
+//   the output are short: 16->40 32^2 13.4 / 17.0, 24->64 32^2 18.6 / 19.9,
+//   16->128 1x1 64^2 15.4 / 19.3, but 64->64 32^2 79 / 27, 48->64 64^2 138 / 68.
+bool split_conv_better(const SlabConv& s) {
+    const int64_t taps = (int64_t)s.kh * s.kw, K = s.C * taps, px = s.N * s.OH * s.OW;
+    if (taps == 9 && s.kh == 3 && s.stride == 1 && s.OH == s.H && s.OW == s.W && s.H <= 16 && s.W <= 16 &&
+        s.C % 16 == 0 && s.M % 32 == 0) {
+        const int64_t cus = num_cus();
+        const double small = s.W % 2 == 0 ? (double)((s.N * (s.M / 32) + cus - 1) / cus) * (4.5 + 0.225 * s.C)
+                                          : (double)((s.N * (s.M / 16) + cus - 1) / cus) * (3.5 + 0.165 * s.C);
+        double split;
+        split_tile_for(s.M, px, K, 1, &split);
+        return split + 7.0 < small;  // (packing the weights, staging the windows)
+    }
+    return K > 32 && !(taps > 1 && K <= 448 && (((s.M <= 48 || (s.stride == 1 && s.M <= 64)) && px <= 32768) ||
+                                    (s.stride == 1 && px <= 16384)));
+}
+
+// Whether the chunk-pipelined backward (pipe_backward, where its geometry
+// holds) is ahead of the split tiles: narrow layers, while a round of its
+// workgroups does not outlast the images' own work. Both gradients, pipelined
+// against split (us): N 64 32->64 14^2 28 / 44, 64->64 14^2 31 / 45, N 256
+// 64->64 14^2 92 / 89, 8^2 79 / 42, N 64 128->128 14^2 114 / 93, 8^2 96 / 51.
+// The weight gradient alone is ahead with enough images: N 64 64->64 14^2
+// 28 / 29, N 8 25 / 15.
+bool pipe_backward_better(const SlabWgrad& w, bool dinput) {
+    return w.C <= 64 && w.M <= 64 && (w.N <= 128 || w.H * w.W > 100) && (dinput || w.N >= 64);
+}
+
+// Whether the slab pair is: narrow layers over small images, where one launch
+// of both gradients fills the chip that neither does alone. Pair against split
+// (us): N 64 16->32 8^2 16 / 21, 16^2 30 / 26, N 256 14^2 31 / 41, N 64 32->64
+// 16^2 33 / 41, 7^2 35 / 29.
+bool slab_pair_better(const SlabWgrad& w) {
+    if (w.H > 16 || w.W > 16 || w.kh * w.kw > 9 || w.stride != 1) return false;
+    if (w.C * w.M <= 512) return w.H * w.W <= 64 || (w.N > 128 && w.H * w.W <= 196);
+    return w.C * w.M <= 2048 && w.H * w.W > 196 && w.N <= 128;
+}
+
 // dinput += the stride-1 input gradient as a slab convolution of the output
 // gradient with the flipped, channel-transposed weights (padding k-1-pad).
 // With `wg`, the weight gradient it describes runs in the same launch when
-// both fit their slab kernels (*wg_done is then set).
+// both fit one of the kernels that take the two (*wg_done is then set).
 int slab_dgrad(float* dinput, const float* grad, const float* weight, int64_t N, int64_t c_in,
                int64_t in_h, int64_t in_w, int64_t c_out, int64_t kh, int64_t kw, int64_t pad,
                const ConvDims& d, const SlabWgrad* wg, bool* wg_done, float beta) {
@@ -1298,30 +1345,25 @@ int slab_dgrad(float* dinput, const float* grad, const float* weight, int64_t N,
     s.OW = (int)in_w;
     s.flip = true;
     s.beta = beta;
+    int rc;
     if (wg) {
         // with the weight gradient: both in one launch
-        int rc = pipe_backward(&s, *wg);
+        rc = pipe_backward_better(*wg, true) ? pipe_backward(&s, *wg) : kSlabUnsupported;
+        if (rc == kSlabUnsupported && slab_pair_better(*wg)) rc = slab_backward_pair(s, *wg);
         if (rc != kSlabUnsupported) {
             *wg_done = rc == NRS_OK;
             return rc;
         }
-        rc = slab_backward_pair(s, *wg);
-        if (rc != kSlabUnsupported) {
-            *wg_done = rc == NRS_OK;
-            return rc;
-        }
-    } else {
-        // small 3x3 images: Winograd F(2x2, 3x3) over the flipped weights,
-        // else the gradient image resident in LDS, the weights flipped while
-        // they are staged (no packing launch)
-        int rc = wino_conv(s);
-        if (rc != kSlabUnsupported) return rc;
-        rc = pipe_conv(s);
-        if (rc != kSlabUnsupported) return rc;
-        rc = img_conv(s);
-        if (rc != kSlabUnsupported) return rc;
     }
-    return slab_conv(s);
+    if (split_conv_better(s) && (rc = split_conv(s)) != kSlabUnsupported) return rc;
+    // small 3x3 images: Winograd F(2x2, 3x3) over the flipped weights,
+    // else the gradient image resident in LDS, the weights flipped while
+    // they are staged (no packing launch)
+    if ((rc = wino_conv(s)) != kSlabUnsupported) return rc;
+    if ((rc = pipe_conv(s)) != kSlabUnsupported) return rc;
+    if ((rc = img_conv(s)) != kSlabUnsupported) return rc;
+    if ((rc = slab_conv(s)) != kSlabUnsupported) return rc;
+    return split_conv(s);
 }
 
 }  // namespace
@@ -1714,6 +1756,10 @@ int nrs_conv2d_forward(float* out, const float* input, const float* weight, cons
         s.OH = (int)d.out_h;
         s.OW = (int)d.out_w;
         if (c_out <= INT32_MAX && d.out_h <= INT32_MAX && d.out_w <= INT32_MAX) {
+            if (nrs::split_conv_better(s)) {
+                rc = nrs::split_conv(s);
+                if (rc != nrs::kSlabUnsupported) return rc;
+            }
             // small "same" 3x3 images: Winograd F(2x2, 3x3) on the matrix
             // cores, else the whole image resident in LDS
             rc = nrs::wino_conv(s);
@@ -1723,6 +1769,8 @@ int nrs_conv2d_forward(float* out, const float* input, const float* weight, cons
             rc = nrs::img_conv(s);
             if (rc != nrs::kSlabUnsupported) return rc;
             rc = nrs::slab_conv(s);
+            if (rc != nrs::kSlabUnsupported) return rc;
+            rc = nrs::split_conv(s);
             if (rc != nrs::kSlabUnsupported) return rc;
         }
     }
@@ -1789,12 +1837,13 @@ int nrs_conv2d_backward_ex(float* dinput, float* dweight, float* dbias, const fl
     NRS_ARG_CHECK(kh < 32768 && kw < 32768 && c_in * in_h * in_w <= INT32_MAX &&
                       c_out * d.out_h * d.out_w <= INT32_MAX && c_out * kh * kw <= INT32_MAX,
                   "conv2d: kernel or image too large");
-    // the slab weight gradient's arguments (it runs beside a slab input
-    // gradient when both fit, else on its own below)
+    // the weight gradient's arguments (a small image's runs beside its input
+    // gradient, others on their own below)
     nrs::SlabWgrad w;
-    const bool slab_w = dweight && col_h > nrs::kDirectTaps && c_in <= INT32_MAX &&
-                        c_out <= INT32_MAX && in_h <= INT32_MAX && in_w <= INT32_MAX;
-    if (slab_w) {
+    const bool fits_w = dweight && c_in <= INT32_MAX && c_out <= INT32_MAX &&
+                        in_h <= INT32_MAX && in_w <= INT32_MAX;
+    const bool slab_w = fits_w && col_h > nrs::kDirectTaps;
+    if (fits_w) {
         w.x = input;
         w.g = grad;
         w.dw = dweight;
@@ -1894,13 +1943,21 @@ int nrs_conv2d_backward_ex(float* dinput, float* dweight, float* dbias, const fl
         f.OW = (int)d.out_w;
         f.beta = beta_params;
         if ((rc = nrs::few_taps_wgrad(f)) != nrs::kSlabUnsupported) return rc;
+        if (fits_w && (rc = nrs::split_wgrad(w)) != nrs::kSlabUnsupported) return rc;
+        // (a bias gradient alone, or tensors past the split tiles' 2 GiB)
         return nrs::small_wgrad(dweight, dbias, grad, input, d, beta_params);
     }
     if (slab_w) {
+        if (nrs::pipe_backward_better(w, false) &&
+            (rc = nrs::pipe_backward(nullptr, w)) != nrs::kSlabUnsupported)
+            return rc;
+        // (16->32 of 256 7x7 images: 18 us split, 15 from the slabs)
+        if (!(w.N > 128 && nrs::slab_pair_better(w)) &&
+            (rc = nrs::split_wgrad(w)) != nrs::kSlabUnsupported)
+            return rc;
         // input slab and gradient rows staged in LDS, reduction on the matrix
-        // cores, per-slice partials summed in a fixed order
-        rc = nrs::pipe_backward(nullptr, w);
-        if (rc != nrs::kSlabUnsupported) return rc;
+        // cores, per-slice partials summed in a fixed order (also tensors past
+        // the split tiles' 2 GiB)
         rc = nrs::slab_wgrad(w);
         if (rc != nrs::kSlabUnsupported) return rc;
     }

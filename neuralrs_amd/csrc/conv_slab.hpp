@@ -92,6 +92,12 @@ struct PipeLower {
 };
 int pipe_backward(const SlabConv* d, const SlabWgrad& w, const PipeLower* lo = nullptr);
 
+// The convolution and the weight and bias gradient as implicit GEMMs on the
+// split tiles (conv_split.hip); kSlabUnsupported (launching nothing) for
+// shapes outside their limits.
+int split_conv(const SlabConv& s);
+int split_wgrad(const SlabWgrad& s);
+
 // Weight and bias gradient of a convolution with c_in*kh*kw <= 15 taps and at
 // most 64 output channels, on the matrix cores (conv_few_taps.hip): dw += and
 // db += (either may be null). Returns kSlabUnsupported (launching nothing)

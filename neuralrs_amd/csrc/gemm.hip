@@ -416,6 +416,30 @@ bool split_eligible(const GemmCall& c) {
            lda < (1 << 21) && ldb < (1 << 21) && (!c.sum_row || c.layout == NRS_TN);
 }
 
+}  // namespace
+
+// The tile of the least estimated time for an unsplit product, and that time
+// in us.
+int split_tile_for(int64_t M, int64_t N, int64_t K, int64_t batch, double* time) {
+    int best = S64x64;
+    double least = 1e30;
+    for (int t = 0; t < S_COUNT; ++t) {
+        const SplitShape& s = kSplitShapes[t];
+        const int64_t per_cu = cdiv(cdiv(M, s.bm) * cdiv(N, s.bn) * batch, (int64_t)num_cus());
+        const double steps = (double)(cdiv(K, s.bk) * s.bk) / 32.0;
+        const double est =
+            (double)per_cu * (steps * (per_cu > 1 ? s.shared : s.alone) + s.fixed);
+        if (est < least) {
+            least = est;
+            best = t;
+        }
+    }
+    if (time) *time = least;
+    return best;
+}
+
+namespace {
+
 // The group kernel takes any dense product the split GEMM's addressing and
 // row of ones allow.
 bool groupable(const GemmCall& c) {
@@ -425,8 +449,8 @@ bool groupable(const GemmCall& c) {
            ldb < (1 << 21) && (!c.sum_row || c.layout == NRS_TN);
 }
 
-// The tile of the least estimated time. Outputs of few 64x64 tiles over a
-// long reduction are split over K as plan_gemm splits them.
+// Outputs of few 64x64 tiles over a long reduction are split over K as
+// plan_gemm splits them, others take one tile's time.
 Plan plan_split(const GemmCall& c) {
     const int64_t M = c.M + (c.sum_row ? 1 : 0), N = c.N, K = c.K;
     const int64_t cus = num_cus();
@@ -439,19 +463,7 @@ Plan plan_split(const GemmCall& c) {
         const int64_t kps = cdiv(cdiv(K, slices), 32) * 32;
         return Plan{S64x64, (int)cdiv(K, kps), kps, 0};
     }
-    Plan best{S64x64, 1, K, 0};
-    double least = 1e30;
-    for (int t = 0; t < S_COUNT; ++t) {
-        const SplitShape& s = kSplitShapes[t];
-        const int64_t wgs = cdiv(M, s.bm) * cdiv(N, s.bn) * c.batch, per_cu = cdiv(wgs, cus);
-        const double steps = (double)(cdiv(K, s.bk) * s.bk) / 32.0;
-        const double step = per_cu > 1 ? s.shared : s.alone;
-        const double est = (double)per_cu * (steps * step + s.fixed);
-        if (est < least) {
-            least = est;
-            best.tile = t;
-        }
-    }
+    Plan best{split_tile_for(M, N, K, c.batch), 1, K, 0};
     best.k_per_slice = cdiv(K, kSplitShapes[best.tile].bk) * kSplitShapes[best.tile].bk;
     return best;
 }

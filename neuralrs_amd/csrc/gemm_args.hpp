@@ -42,7 +42,6 @@ struct GemmArgs {
 enum SplitTile { S256x256 = 0, S128x128, S64x128, S64x64K, S64x64, S_COUNT };
 using SplitKernel = void (*)(GemmArgs);
 SplitKernel split_kernel(int tile, int layout);
-
 // Problems of one group launch: the C ABI's groups (NRS_GEMM_GROUP_MAX) and
 // the backward of three products sharing their left operand (three input-
 // gradient and three weight-gradient products).

@@ -159,25 +159,46 @@ __device__ __forceinline__ void split_pos(int i, int tid, int& row, int& q) {
 // offset of each of the thread's units there (rows past the operand read its
 // last row: their results are not stored). The k-tile's address is in the
 // buffer's base, so offsets stay below 256 rows of the operand.
-template <int BMN, int BK, bool KC, int NT, int U>
+// (What split_tile asks of an operand: kKC, the order of its units over the
+// threads; kOnes and `ones`, bit i set where unit i is all ones; kMasked, true
+// if load<false> reads zero past the end of k; begin, called before the first
+// unit of a k-tile is loaded; load; at, any one element; and kFix, of a column
+// operand whose loaded units go through fix before they are split.)
+template <int BMN, int BK, bool KC, int NT, int U, bool ONES = false>
 struct SplitOperand {
+    static constexpr bool kKC = KC, kOnes = ONES, kMasked = false, kFix = false;
     const float* base;  // the tile's first row (column) at k = 0
     int64_t ld;
     int off[U];
+    int last;  // last row of the operand in the tile
+    uint32_t ones = 0;
+    int one_row = -1;
 
+    // `one`: the operand row made of ones (-1: none).
     __device__ __forceinline__ void init(const float* X, int64_t ld_, int64_t mn0, int64_t MN,
-                                         int tid) {
+                                         int64_t one, int tid) {
         ld = ld_;
         const int64_t first = min(mn0, MN - 1);
         base = X + (KC ? first * ld : first);
-        const int last = (int)min((int64_t)(BMN - 1), MN - 1 - first);
+        last = (int)min((int64_t)(BMN - 1), MN - 1 - first);
 #pragma unroll
         for (int i = 0; i < U; ++i) {
             int row, q;
             split_pos<BMN, BK, KC, NT>(i, tid, row, q);
             const int mn = min(row, last);
             off[i] = 4 * (KC ? mn * (int)ld + 4 * q : mn + 4 * q * (int)ld);
+            if constexpr (ONES) ones |= (uint32_t)(mn0 + row == one) << i;
         }
+        if constexpr (ONES) one_row = one >= 0 ? (int)(one - mn0) : -1;
+    }
+
+    __device__ __forceinline__ void begin(int64_t, int) {}
+    __device__ __forceinline__ void fix(f32x4 (&)[2], int) const {}
+
+    __device__ __forceinline__ float at(int row, int64_t k) const {
+        const int r = min(row, last);
+        const float x = KC ? base[r * ld + k] : base[k * ld + r];
+        return ONES && row == one_row ? 1.0f : x;
     }
 
     // Loads unit i of the k-tile at k0. PART: elements at or past kend read
@@ -215,13 +236,12 @@ struct SplitOperand {
     }
 };
 
-// The wave's (32 FM) x (32 FN) block at (m0, n0) over [kbeg, kend) on the f32
-// instructions, operands from global memory (the exceptions above: any
-// inputs, no staging, not fast).
-template <int FM, int FN, bool AK, bool BKC>
-__device__ __forceinline__ void f32_block(f32x16 (&acc)[FM][FN], const float* A, const float* B,
-                                       const GemmArgs& p, int64_t m0, int64_t n0, int64_t kbeg,
-                                       int64_t kend, int lane) {
+// The wave's (32 FM) x (32 FN) block at (m0, n0) of the tile over [kbeg, kend)
+// on the f32 instructions, operands element by element from global memory (the
+// exceptions above: any inputs, no staging, not fast).
+template <int FM, int FN, class OA, class OB>
+__device__ __forceinline__ void f32_block(f32x16 (&acc)[FM][FN], const OA& oa, const OB& ob, int m0,
+                                          int n0, int64_t kbeg, int64_t kend, int lane) {
     const int h = lane >> 5, l32 = lane & 31;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -231,20 +251,17 @@ __device__ __forceinline__ void f32_block(f32x16 (&acc)[FM][FN], const float* A,
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 #pragma unroll 1
     for (int64_t k = kbeg; k < kend; k += 2) {
-        const int64_t kk = k + h;
-        const bool ok = kk < kend;
-        const int64_t ks = ok ? kk : kbeg;
+        const bool ok = k + h < kend;
+        const int64_t kk = ok ? k + h : kbeg;
         float a[FM], b[FN];
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
-            const int64_t row = m0 + 32 * i + l32, rr = min(row, p.M - 1);
-            const float x = AK ? A[rr * p.lda + ks] : A[ks * p.lda + rr];
-            a[i] = ok ? (p.sum_row && row == p.M ? 1.0f : x) : 0.0f;
+            const float x = oa.at(m0 + 32 * i + l32, kk);
+            a[i] = ok ? x : 0.0f;
         }
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-            const int64_t col = min(n0 + 32 * j + l32, p.N - 1);
-            const float x = BKC ? B[col * p.ldb + ks] : B[ks * p.ldb + col];
+            const float x = ob.at(n0 + 32 * j + l32, kk);
             b[j] = ok ? x : 0.0f;
         }
 #pragma unroll
@@ -255,9 +272,12 @@ __device__ __forceinline__ void f32_block(f32x16 (&acc)[FM][FN], const float* A,
     }
 }
 
-template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int KS, bool TWO, bool AK, bool BKC>
-__device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, int64_t m0, int64_t n0,
-                                           int64_t kbeg, int64_t kend, int slice, int64_t batch) {
+// The tile at (m0, n0) over [kbeg, kend) of the product of the initialised
+// operands oa (rows) and ob (columns), stored by p's epilogue.
+template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int KS, bool TWO, class OA, class OB>
+__device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& oa, OB& ob,
+                                           int64_t m0, int64_t n0, int64_t kbeg, int64_t kend,
+                                           int slice, int64_t batch) {
     using C_ = SplitCfg<BM, BN, BK, WAVES_M, WAVES_N, KS>;
     constexpr int FM = C_::FM, FN = C_::FN, NT = C_::NT;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -266,24 +286,6 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, int64
     const int wave = wave_id - kset * (WAVES_M * WAVES_N);
     const int h = lane >> 5, l32 = lane & 31;
     const int wm0 = (wave / WAVES_N) * C_::WM, wn0 = (wave % WAVES_N) * C_::WN;
-    const float* A = p.A + batch * p.sA;
-    const float* B = p.B + batch * p.sB;
-
-    SplitOperand<BM, BK, AK, NT, C_::UA> oa;
-    SplitOperand<BN, BK, BKC, NT, C_::UB> ob;
-    oa.init(A, p.lda, m0, p.M, tid);
-    ob.init(B, p.ldb, n0, p.N, tid);
-    uint32_t ones = 0;
-    if constexpr (!AK) {
-        if (p.sum_row) {
-#pragma unroll
-            for (int i = 0; i < C_::UA; ++i) {
-                int row, q;
-                split_pos<BM, BK, AK, NT>(i, tid, row, q);
-                ones |= (uint32_t)(m0 + row == p.M) << i;
-            }
-        }
-    }
 
     f32x16 acc[FM][FN], lo[TWO ? FM : 1][TWO ? FN : 1];
 #pragma unroll
@@ -301,11 +303,16 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, int64
     const int ntiles = (int)((kend - kbeg + BK - 1) / BK);
     // Tile t of the slice goes through the staging registers into LDS buffer
     // t % 2. Units are numbered A's first.
-    const int nfull = (int)((kend - kbeg) / BK);
+    constexpr bool kMasked = OA::kMasked && OB::kMasked;
+    const int nfull = kMasked ? ntiles : (int)((kend - kbeg) / BK);
     constexpr int kUnits = C_::UA + C_::UB;
     auto load_unit = [&](int t, int un, auto part) {
         constexpr bool PART = decltype(part)::value;
         const int64_t k0 = kbeg + (int64_t)t * BK;
+        if (un == 0) {
+            oa.begin(k0, tid);
+            ob.begin(k0, tid);
+        }
         if (un < C_::UA)
             oa.template load<PART>(ra[un], un, k0, kend, tid);
         else
@@ -330,14 +337,16 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, int64
         constexpr int x = decltype(xc)::value, un = x / kSplitSteps;
         constexpr bool in_a = un < C_::UA;
         constexpr int i = in_a ? un : un - C_::UA;
+        if constexpr (!in_a && OB::kFix && x % kSplitSteps == 0) ob.fix(rb[i], i);
         st.template step<x % kSplitSteps>(in_a ? ra[i] : rb[i], sticky,
-                                          !AK && in_a && ((ones >> i) & 1u));
+                                          in_a ? OA::kOnes && ((oa.ones >> i) & 1u)
+                                               : OB::kOnes && ((ob.ones >> i) & 1u));
         if constexpr (x % kSplitSteps == kSplitSteps - 1) {
             int row, q;
             if (in_a)
-                split_pos<BM, BK, AK, NT>(i, tid, row, q);
+                split_pos<BM, BK, OA::kKC, NT>(i, tid, row, q);
             else
-                split_pos<BN, BK, BKC, NT>(i, tid, row, q);
+                split_pos<BN, BK, OB::kKC, NT>(i, tid, row, q);
             u32x4* dst = smem + (t & 1) * C_::STAGE + (in_a ? 0 : 3 * C_::PLANE_A);
             const int at = split_unit<BK>(row, q);
 #pragma unroll
@@ -506,11 +515,24 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, int64
                 for (int r = 0; r < 16; ++r) small |= fabsf(out[i][j][r]) < 0x1p-70f;
     }
     if (__any(small || finite != 0.0f))
-        f32_block<FM, FO, AK, BKC>(out, A, B, p, m0 + wm0, n0 + wo0, kbeg, kend, lane);
+        f32_block<FM, FO>(out, oa, ob, wm0, wo0, kbeg, kend, lane);
 
     const TileOut<FO> to = tile_out<BM, BN, FO>(p, m0, n0, wm0, wo0, h, l32, slice, batch);
     const float none[1][1][16] = {};
     tile_store<FM, FO, false>(p, to, out, none, n0 + wo0 + l32);
+}
+
+// split_tile of a dense problem.
+template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int KS, bool TWO, bool AK, bool BKC>
+__device__ __forceinline__ void split_dense(const GemmArgs& p, u32x4* smem, int64_t m0, int64_t n0,
+                                            int64_t kbeg, int64_t kend, int slice, int64_t batch) {
+    using C_ = SplitCfg<BM, BN, BK, WAVES_M, WAVES_N, KS>;
+    SplitOperand<BM, BK, AK, C_::NT, C_::UA, !AK> oa;
+    SplitOperand<BN, BK, BKC, C_::NT, C_::UB> ob;
+    oa.init(p.A + batch * p.sA, p.lda, m0, p.M, p.sum_row ? p.M : -1, threadIdx.x);
+    ob.init(p.B + batch * p.sB, p.ldb, n0, p.N, -1, threadIdx.x);
+    split_tile<BM, BN, BK, WAVES_M, WAVES_N, KS, TWO>(p, smem, oa, ob, m0, n0, kbeg, kend, slice,
+                                                      batch);
 }
 
 template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int KS, bool TWO, bool AK, bool BKC>
@@ -523,7 +545,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * KS, 2) void gemm_split_ker
     int tm, tn;
     tile_coords(p, bid, tm, tn);
     const int64_t kbeg = (int64_t)slice * p.k_per_slice;
-    split_tile<BM, BN, BK, WAVES_M, WAVES_N, KS, TWO, AK, BKC>(p, smem, (int64_t)tm * BM, (int64_t)tn * BN,
+    split_dense<BM, BN, BK, WAVES_M, WAVES_N, KS, TWO, AK, BKC>(p, smem, (int64_t)tm * BM, (int64_t)tn * BN,
                                                       kbeg, min(p.K, kbeg + p.k_per_slice), slice,
                                                       blockIdx.z);
 }
@@ -558,15 +580,15 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 3) void gemm_split_group_ke
     const int64_t kbeg = (int64_t)slice * p.k_per_slice, kend = min(p.K, kbeg + p.k_per_slice);
     switch (g.layout[q]) {
         case NRS_NN:
-            split_tile<BM, BN, BK, WAVES_M, WAVES_N, 1, true, true, false>(p, smem, m0, n0, kbeg,
+            split_dense<BM, BN, BK, WAVES_M, WAVES_N, 1, true, true, false>(p, smem, m0, n0, kbeg,
                                                                            kend, slice, 0);
             break;
         case NRS_NT:
-            split_tile<BM, BN, BK, WAVES_M, WAVES_N, 1, true, true, true>(p, smem, m0, n0, kbeg,
+            split_dense<BM, BN, BK, WAVES_M, WAVES_N, 1, true, true, true>(p, smem, m0, n0, kbeg,
                                                                           kend, slice, 0);
             break;
         default:
-            split_tile<BM, BN, BK, WAVES_M, WAVES_N, 1, true, false, false>(p, smem, m0, n0, kbeg,
+            split_dense<BM, BN, BK, WAVES_M, WAVES_N, 1, true, false, false>(p, smem, m0, n0, kbeg,
                                                                             kend, slice, 0);
             break;
     }

@@ -1,0 +1,140 @@
+"""Convolutions on the split tiles (conv_split.hip), against f64.
+
+Shapes take every tile and every staging form where it can go wrong: channels
+that are and are not whole k steps, ragged channel and pixel tiles, rows of
+whole quads (128-bit loads, moved one pixel at the image's edges) and ragged
+rows, strides, padding 0 and past 1, 1x1 and 5x5 kernels, few-channel weight
+gradients, pointers off 16 bytes.
+
+Bars: bit-exact where every product and partial sum is an integer below 2^24
+(one operand of up to 16 bits, so that every piece carries bits); against f64,
+|y - y64| <= (6 K / 16 + 72) * 2^-24 * (|x| * |w|) element by element: each
+instruction rounds once, six products a step of 16, a weight gradient's partial
+sums (at most 64 long a chain) and its beta round too.
+"""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+from kat import int_matrix
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # n, c_in, c_out, h, w, kh, kw, stride, pad
+    (2, 64, 64, 24, 24, 3, 3, 1, 1),     # whole k steps and tiles, 128-bit window loads
+    (3, 64, 72, 17, 19, 3, 3, 1, 1),     # ragged rows, ragged channel tile
+    (9, 36, 65, 21, 20, 3, 3, 1, 1),     # channels across k steps, pixels across images
+    (40, 128, 128, 21, 21, 3, 3, 1, 1),  # 128x128 tiles
+    (2, 64, 48, 23, 20, 3, 3, 1, 0),     # no padding
+    (2, 64, 40, 18, 18, 3, 3, 1, 2),     # padding past 1
+    (2, 64, 64, 20, 20, 5, 5, 1, 2),
+    (2, 40, 72, 30, 28, 1, 1, 1, 0),
+    (2, 64, 36, 31, 33, 3, 3, 2, 1),
+    (2, 32, 64, 32, 32, 3, 3, 2, 1),     # strided, rows of whole quads
+    (2, 64, 64, 12, 40, 2, 4, 1, 1),     # kernel and image not square
+    (4, 3, 32, 32, 32, 3, 3, 1, 1),      # weight gradient of 27 columns
+    (4, 3, 96, 30, 29, 3, 3, 2, 1),
+    (2, 1, 96, 28, 28, 3, 3, 1, 1),
+    (2, 16, 20, 40, 40, 3, 3, 1, 1),     # 145 columns, 20 rows
+    # a few k steps in all (not a "same" layer: Winograd's sums, which such small
+    # ones take, cancel, and its error has no bound element by element)
+    (1, 16, 32, 5, 6, 3, 3, 1, 0),
+    (1, 9, 70, 1, 4, 3, 3, 1, 1),        # one output row of one quad
+    (3, 256, 160, 7, 7, 3, 3, 1, 1),
+]
+IDS = lambda s: "x".join(map(str, s))
+
+
+def device(hip, x, offset):
+    buf = hip.DeviceBuffer.from_host(np.concatenate([np.zeros(offset, np.float32), x.ravel()]))
+    return buf, buf.ptr + 4 * offset
+
+
+def reference(shape, x, w, b, g):
+    n, ci, co, h, wd, kh, kw, s, p = shape
+    tx, tw, tb = (torch.from_numpy(v.astype(np.float64)).requires_grad_() for v in (x, w, b))
+    y = F.conv2d(tx, tw, tb, stride=s, padding=p)
+    y.backward(torch.from_numpy(g.astype(np.float64)))
+    return [v.detach().numpy() for v in (y, tx.grad, tw.grad, tb.grad)]
+
+
+def run(hip, shape, x, w, b, g, old, beta_in, beta_par, offset=0, dinput=True):
+    n, ci, co, h, wd, kh, kw, s, p = shape
+    dims = (n, ci, h, wd, co, kh, kw, s, p)
+    keep = [device(hip, v, offset) for v in (x, w, b, g)]
+    px, pw, pb, pg = (k[1] for k in keep)
+    y = hip.DeviceBuffer.from_host(np.full(g.size, np.nan, np.float32))
+    hip.call("nrs_conv2d_forward", y.ptr, px, pw, pb, *dims)
+    dx, dw, db = (hip.DeviceBuffer.from_host(v) for v in old)
+    hip.call("nrs_conv2d_backward_ex", dx.ptr if dinput else None, dw.ptr, db.ptr, pg, px, pw, *dims,
+             beta_in, beta_par)
+    return y.to_host(g.shape), dx.to_host(x.shape), dw.to_host(w.shape), db.to_host(b.shape)
+
+
+def sizes(shape):
+    n, ci, co, h, w, kh, kw, s, p = shape
+    oh, ow = (h + 2 * p - kh) // s + 1, (w + 2 * p - kw) // s + 1
+    return (n, ci, h, w), (co, ci, kh, kw), (co,), (n, co, oh, ow)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=IDS)
+def test_exact_integers_all_pieces(hip, shape):
+    sx, sw, sb, sg = sizes(shape)
+    rng = np.random.default_rng(sum(shape))
+    longest = max(sw[1] * sw[2] * sw[3], sw[0] * sw[2] * sw[3], sg[0] * sg[2] * sg[3])
+    bits = min(16, 23 - int(np.ceil(np.log2(longest))))
+    wide = lambda s: int_matrix(rng, s, -2 ** bits + 1, 2 ** bits - 1)
+    sign = lambda s: int_matrix(rng, s, -1, 1)
+    # (the input gradient is g * w, the weight gradient g * x)
+    for offset, (mx, mw, mg) in enumerate([(wide, sign, sign), (sign, wide, sign), (sign, sign, wide)]):
+        x, w, b, g = mx(sx), mw(sw), sign(sb), mg(sg)
+        old = [sign(sx), sign(sw), sign(sb)]
+        got = run(hip, shape, x, w, b, g, old, 1.0, 1.0, offset)
+        want = reference(shape, x, w, b, g)
+        for k, name in enumerate(("output", "input gradient", "weight gradient", "bias gradient")):
+            assert np.array_equal(got[k].astype(np.float64), want[k] + (old[k - 1] if k else 0)), name
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=IDS)
+def test_f64_error(hip, shape):
+    sx, sw, sb, sg = sizes(shape)
+    rng = np.random.default_rng(3 + sum(shape))
+    # magnitudes over nine decades, one value in three zero
+    make = lambda s: (rng.standard_normal(s) * 10.0 ** rng.integers(-6, 4, s) *
+                      (rng.random(s) > 0.33)).astype(np.float32)
+    x, w, b, g = make(sx), make(sw), make(sb), make(sg)
+    nan = [np.full(s, np.nan, np.float32) for s in (sx, sw, sb)]
+    got = run(hip, shape, x, w, b, g, nan, 0.0, 0.0, dinput=False)
+    grads = run(hip, shape, x, w, b, g, nan, 0.0, 0.0)
+    assert np.isnan(got[1]).all()  # no input gradient asked for
+    want, size = reference(shape, x, w, b, g), reference(shape, *map(np.abs, (x, w, b, g)))
+    ks = (sw[1] * sw[2] * sw[3], sw[0] * sw[2] * sw[3], sg[0] * sg[2] * sg[3], sg[0] * sg[2] * sg[3])
+    for k, name in enumerate(("output", "input gradient", "weight gradient", "bias gradient")):
+        bound = (6 * ks[k] / 16 + 72) * 2.0 ** -24 * size[k] + 1e-35
+        for y in ((grads[k],) if k == 1 else (got[k], grads[k])):
+            assert np.all(np.abs(y - want[k]) <= bound), name
+
+
+@pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[1], SHAPES[3], SHAPES[9], SHAPES[11]], ids=IDS)
+def test_infinities_and_nan_stay_where_they_belong(hip, shape):
+    sx, sw, sb, sg = sizes(shape)
+    rng = np.random.default_rng(5 + sum(shape))
+    small = lambda s: int_matrix(rng, s, 1, 4)
+    x, w, b, g = small(sx), small(sw), small(sb), small(sg)
+    x[0, 1, 2, 3], x[-1, 0, -1, -1] = np.inf, np.float32(3.4028235e38)
+    # (the values that are not finite meet no padding: a lowering's padding zeros
+    # times them are NaN, where torch has no such term)
+    w[5, 0, 1, 1] = np.nan
+    w[3, 1, 1, 1] = 2.0 ** -100
+    g[0, 2, 1, 1], g[-1, 1, -2, -2] = -np.inf, np.nan
+    old = [np.zeros(s, np.float32) for s in (sx, sw, sb)]
+    got = run(hip, shape, x, w, b, g, old, 0.0, 0.0)
+    want = reference(shape, x, w, b, g)
+    for k in range(4):
+        with np.errstate(over="ignore"):
+            f = want[k].astype(np.float32)
+        bad = ~np.isfinite(f)
+        assert not np.isfinite(got[k][bad]).any()
+        ok = ~bad
+        assert np.all(np.abs(got[k][ok] - f[ok]) <= 1e-4 * np.abs(f[ok]) + 1e-30)
