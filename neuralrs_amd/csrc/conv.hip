@@ -1282,13 +1282,26 @@ int small_wgrad(float* dweight, float* dbias, const float* grad, const float* in
 // - the slab kernel is ahead by its one launch less where the reduction and
 //   the output are short: 16->40 32^2 13.4 / 17.0, 24->64 32^2 18.6 / 19.9,
 //   16->128 1x1 64^2 15.4 / 19.3, but 64->64 32^2 79 / 27, 48->64 64^2 138 / 68.
+//   Under 16 channels of 9 taps it stays ahead over any number of pixels (64
+//   outputs, N 256: 16 channels 20^2 32.0 / 36.9, 8 channels 16^2 15.0 / 18.7),
+//   under 24 up to the 65536 of N 256 16^2 (21.4 / 26.5), and 64->64 1x1 20^2
+//   (N 256 23 / 25). Over few pixels a long reduction leaves the split tiles a
+//   chain of k steps on part of the chip: 32->64 5x5 N 64 10^2 17.5 / 22.7,
+//   64->64 stride 2 N 64 10^2 15.2 / 17.5.
+// (Two workgroups of the odd images' kernel fit a CU: 16->64 5^2 N 128 takes
+// one round, 6.6 against 12.3.)
 bool split_conv_better(const SlabConv& s) {
     const int64_t taps = (int64_t)s.kh * s.kw, K = s.C * taps, px = s.N * s.OH * s.OW;
+    if (s.M <= 64 && (taps == 1 ? K <= 64
+                                : K <= 144 ? s.stride == 1 || px > 32768
+                                : K <= 216 && s.stride == 1 ? px <= 65536
+                                : taps > 9 ? px <= 8192 : s.stride > 1 && K <= 576 && px <= 2048))
+        return false;
     if (taps == 9 && s.kh == 3 && s.stride == 1 && s.OH == s.H && s.OW == s.W && s.H <= 16 && s.W <= 16 &&
         s.C % 16 == 0 && s.M % 32 == 0) {
         const int64_t cus = num_cus();
         const double small = s.W % 2 == 0 ? (double)((s.N * (s.M / 32) + cus - 1) / cus) * (4.5 + 0.225 * s.C)
-                                          : (double)((s.N * (s.M / 16) + cus - 1) / cus) * (3.5 + 0.165 * s.C);
+                                          : (double)((s.N * (s.M / 16) + 2 * cus - 1) / (2 * cus)) * (3.5 + 0.165 * s.C);
         double split;
         split_tile_for(s.M, px, K, 1, &split);
         return split + 7.0 < small;  // (packing the weights, staging the windows)
@@ -1303,19 +1316,47 @@ bool split_conv_better(const SlabConv& s) {
 // against split (us): N 64 32->64 14^2 28 / 44, 64->64 14^2 31 / 45, N 256
 // 64->64 14^2 92 / 89, 8^2 79 / 42, N 64 128->128 14^2 114 / 93, 8^2 96 / 51.
 // The weight gradient alone is ahead with enough images: N 64 64->64 14^2
-// 28 / 29, N 8 25 / 15.
+// 28 / 29, N 8 25 / 15, N 256 32->64 8^2 19 / 22, 10^2 22 / 31, 64->64 10^2
+// 36 / 40, 8^2 32 / 27.
 bool pipe_backward_better(const SlabWgrad& w, bool dinput) {
-    return w.C <= 64 && w.M <= 64 && (w.N <= 128 || w.H * w.W > 100) && (dinput || w.N >= 64);
+    if (w.C > 64 || w.M > 64) return false;
+    if (dinput) return w.N <= 128 || w.H * w.W > 100;
+    return w.N >= 64 && (w.N <= 128 || w.H * w.W >= 100 || w.C <= 32);
+}
+
+// Whether the slab weight gradient on its own is: many small images, above all
+// of rows that are no whole quads, whose pixels the split tiles gather one by
+// one. Slab against split (us): N 256 16->32 7^2 15 / 18; 10^2 N 128 32->32
+// 18 / 21, N 256 16->64 20 / 26, N 64 32->32 17 / 15; 9^2 N 100 32->32 17 / 19;
+// 14^2 N 128 24->64 25 / 28,
+// N 256 16->64 26 / 32, 64->32 59 / 50; of quads, 12^2 N 256 32->32 28 / 25.
+bool slab_wgrad_better(const SlabWgrad& w) {
+    const int64_t pixels = (int64_t)w.H * w.W;
+    if (w.kh * w.kw > 9 || w.stride != 1 || pixels > 196) return false;
+    if (w.N > 128 && w.C * w.M <= 512) return true;
+    return w.OW % 4 != 0 && pixels >= 81 && w.C >= 16 && w.C <= 32 && w.N >= 96;
 }
 
 // Whether the slab pair is: narrow layers over small images, where one launch
-// of both gradients fills the chip that neither does alone. Pair against split
-// (us): N 64 16->32 8^2 16 / 21, 16^2 30 / 26, N 256 14^2 31 / 41, N 64 32->64
-// 16^2 33 / 41, 7^2 35 / 29.
+// of both gradients fills the chip that neither does alone. Up to 14x14 an
+// image is one band, and the pair's time is mostly its launches' until images
+// times products, the input channels counted twice (they are the output rows of
+// one half and the columns of the other), outgrow the chip. Pair against split
+// (us): 14^2 N 128 16->64 30 / 41, 32->32 30 / 39, 64->32 51 / 47; 10^2 N 64
+// 8->64 19 / 28, N 256 16->64 28 / 41, 64->16 49 / 46; 8^2 N 64 32->32 17 / 23,
+// N 256 64->20 48 / 40. Larger images come in bands: 16^2 N 64 32->64 33 / 41,
+// 8->64 30 / 29, N 128 43 / 33. Up to 32 input channels the split tiles do not
+// take the input gradient, and on its own over many gradient channels it is one
+// long chain a workgroup: 32->96 N 24 15^2 37 / 66, N 8 40^2 47 / 57.
 bool slab_pair_better(const SlabWgrad& w) {
-    if (w.H > 16 || w.W > 16 || w.kh * w.kw > 9 || w.stride != 1) return false;
-    if (w.C * w.M <= 512) return w.H * w.W <= 64 || (w.N > 128 && w.H * w.W <= 196);
-    return w.C * w.M <= 2048 && w.H * w.W > 196 && w.N <= 128;
+    const int64_t pixels = (int64_t)w.H * w.W, size = (int64_t)w.C * w.C * w.M * w.N;
+    const int taps = w.kh * w.kw;
+    if (taps > 9 || w.stride != 1) return false;
+    if (taps > 1 && w.M > 64 && w.C > 16 && w.C <= 32 && w.N * pixels <= 16384) return true;
+    if (w.H > 16 || w.W > 16) return false;
+    if (pixels <= (w.OW % 4 ? 225 : 196) && size <= (taps == 1 && pixels <= 100 ? 20 : 15) << 20) return true;
+    if (w.C * w.M <= 512) return pixels <= 64 || (w.N > 128 && pixels <= 196);
+    return w.C * w.M <= 2048 && pixels > 196 && size <= (1 << 22);
 }
 
 // dinput += the stride-1 input gradient as a slab convolution of the output
@@ -1951,9 +1992,7 @@ int nrs_conv2d_backward_ex(float* dinput, float* dweight, float* dbias, const fl
         if (nrs::pipe_backward_better(w, false) &&
             (rc = nrs::pipe_backward(nullptr, w)) != nrs::kSlabUnsupported)
             return rc;
-        // (16->32 of 256 7x7 images: 18 us split, 15 from the slabs)
-        if (!(w.N > 128 && nrs::slab_pair_better(w)) &&
-            (rc = nrs::split_wgrad(w)) != nrs::kSlabUnsupported)
+        if (!nrs::slab_wgrad_better(w) && (rc = nrs::split_wgrad(w)) != nrs::kSlabUnsupported)
             return rc;
         // input slab and gradient rows staged in LDS, reduction on the matrix
         // cores, per-slice partials summed in a fixed order (also tensors past
