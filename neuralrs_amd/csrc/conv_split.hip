@@ -26,7 +26,7 @@
 // of stride 1 unless said):
 //   forward      64->128 32 x 32^2 117 -> 38    128->128 64 x 28^2 225 -> 108
 //                64->64 5x5 32 x 32^2 135 -> 58   64->128 stride 2 32 x 56^2 66 -> 37
-//   wgrad + bias 16->32 32 x 64^2 75 -> 43   64->128 32 x 32^2 122 -> 44
+//   wgrad + bias 16->32 32 x 64^2 75 -> 34   64->128 32 x 32^2 122 -> 44
 //                128->128 64 x 28^2 310 -> 104   3->32 32 x 64^2 121 -> 21
 //                1x1 64->128 32 x 32^2 101 -> 20
 #include <algorithm>
@@ -420,20 +420,32 @@ __global__ __launch_bounds__(64 * kSumWaves) void conv_split_sum_kernel(
 
 using WgradKernel = void (*)(ConvSplitArgs);
 
-template <int BM, int BN, int KS>
+template <int BM, int BN, int WAVES_M, int KS>
 WgradKernel wgrad_form(int form) {
     switch (form) {
-        case 0: return conv_split_wgrad_kernel<BM, BN, 32, 2, 2, KS, false, false>;
-        case 1: return conv_split_wgrad_kernel<BM, BN, 32, 2, 2, KS, true, false>;
-        default: return conv_split_wgrad_kernel<BM, BN, 32, 2, 2, KS, true, true>;
+        case 0: return conv_split_wgrad_kernel<BM, BN, 32, WAVES_M, 2, KS, false, false>;
+        case 1: return conv_split_wgrad_kernel<BM, BN, 32, WAVES_M, 2, KS, true, false>;
+        default: return conv_split_wgrad_kernel<BM, BN, 32, WAVES_M, 2, KS, true, true>;
     }
 }
-WgradKernel wgrad_kernel(int tile, int form) {
-    switch (tile) {
-        case S128x128: return wgrad_form<128, 128, 2>(form);
-        case S64x128: return wgrad_form<64, 128, 1>(form);
-        default: return wgrad_form<64, 64, 1>(form);
-    }
+// Tiles of the weight gradient: `fit` workgroups share a CU (by LDS). Staging
+// a column operand unit costs more than its products, so a tile is as wide as
+// the columns allow, but for at most 32 rows: there half of a 64-row tile's
+// products are padding, and past 128 columns 64-wide tiles also pad less and
+// leave four workgroups a CU to cover each other's gathering. 64x128 against
+// 32x64 (us, with the sum): 16->32 3x3 32 x 64^2 42.0 / 33.5 (145 columns), 16 x
+// 32->32 64^2 35.4 / 28.4, 16 x 128->32 56^2 70.4 / 57.8, 1x1 128->32 32 x 32^2
+// 21.5 / 17.9; one wide tile of columns stays ahead: 8->32 64 x 32^2 (73
+// columns) 19.8 / 20.8, 3->32 32 x 64^2 (28) 21.3 / 23.3.
+struct WgradTile {
+    int bm, bn, threads, fit;
+    WgradKernel kernel;
+};
+WgradTile wgrad_tile(int64_t M, int64_t N, int form) {
+    if (M <= 32 && N > 128) return {32, 64, 128, 4, wgrad_form<32, 64, 1, 1>(form)};
+    if (N <= 64) return {64, 64, 256, 2, wgrad_form<64, 64, 2, 1>(form)};
+    if (M <= 64) return {64, 128, 256, 2, wgrad_form<64, 128, 2, 1>(form)};
+    return {128, 128, 512, 1, wgrad_form<128, 128, 2, 2>(form)};
 }
 
 }  // namespace
@@ -525,12 +537,10 @@ int split_wgrad(const SlabWgrad& s) {
     a.div_taps = make_fastdiv((uint32_t)taps);
     a.div_rowq = make_fastdiv((uint32_t)row_q);
     a.div_oh = make_fastdiv((uint32_t)s.OH);
-    // staging a column operand unit costs more than its products: the tile is
-    // as wide as the columns allow
-    const int tile = g.N <= 64 ? S64x64 : (s.M > 64 ? S128x128 : S64x128);
-    const int bm = tile == S128x128 ? 128 : 64, bn = tile == S64x64 ? 64 : 128;
-    g.tiles_m = (int)cdiv(s.M, bm);
-    g.tiles_n = (int)cdiv(g.N, bn);
+    const int form = s.OW % 4 ? 0 : (s.stride == 1 && s.pad <= 1 && s.W >= 4 ? 2 : 1);
+    const WgradTile t = wgrad_tile(s.M, g.N, form);
+    g.tiles_m = (int)cdiv(s.M, t.bm);
+    g.tiles_n = (int)cdiv(g.N, t.bn);
     const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n, ksteps = g.K / 32;
     // One round of workgroups (one 128x128 tile fits a CU, two of the others),
     // at most 256 slices, and of a short reduction as many as balance a slice's
@@ -538,7 +548,7 @@ int split_wgrad(const SlabWgrad& s) {
     // outputs): 16->32 8 x 8x8, 16 steps, 13.0 us with 4 steps a slice, 9.4 with
     // 1; 64 x 14x14, 392 steps, 15.4 with 4, 17.2 with 2; 32->48 8 x 30x30, 240
     // steps, 16.6 with 4, 19.3 with 2.
-    const int64_t round = (tile == S128x128 ? 1 : 2) * (int64_t)num_cus();
+    const int64_t round = t.fit * (int64_t)num_cus();
     const double add = 0.03 + 1e-6 * (double)(s.M * g.N), step = 1.1;
     const int64_t least = std::max<int64_t>(1, std::llround(std::sqrt((double)ksteps * add / step)));
     int64_t slices = std::max<int64_t>(1, std::min({round / tiles, cdiv(ksteps, least), (int64_t)256}));
@@ -547,8 +557,7 @@ int split_wgrad(const SlabWgrad& s) {
     g.partial = workspace(sizeof(float) * (size_t)(slices * s.M * g.N), 3);
     if (!g.partial) return NRS_ERR_ALLOC;
     const dim3 grid((unsigned)tiles, (unsigned)slices);
-    const int form = s.OW % 4 ? 0 : (s.stride == 1 && s.pad <= 1 && s.W >= 4 ? 2 : 1);
-    hipLaunchKernelGGL(wgrad_kernel(tile, form), grid, dim3(tile == S128x128 ? 512 : 256), 0, stream(), a);
+    hipLaunchKernelGGL(t.kernel, grid, dim3(t.threads), 0, stream(), a);
     NRS_LAUNCH_CHECK("conv2d weight gradient (split)");
     const int64_t total = s.M * g.N;
     hipLaunchKernelGGL(conv_split_sum_kernel, dim3((unsigned)cdiv(total, 64)), dim3(64 * kSumWaves), 0,

@@ -37,6 +37,11 @@ SHAPES = [  # n, c_in, c_out, h, w, kh, kw, stride, pad
     (4, 3, 96, 30, 29, 3, 3, 2, 1),
     (2, 1, 96, 28, 28, 3, 3, 1, 1),
     (2, 16, 20, 40, 40, 3, 3, 1, 1),     # 145 columns, 20 rows
+    (2, 16, 32, 41, 39, 3, 3, 1, 1),     # 32-row tiles full, ragged rows of pixels
+    (4, 128, 1, 24, 24, 1, 1, 1, 0),     # one channel, 129 columns
+    (2, 8, 33, 40, 40, 4, 4, 1, 1),      # a row and a column past them (33, 129)
+    (4, 8, 32, 48, 48, 4, 4, 2, 1),      # 129 columns, strided rows of whole quads
+    (4, 24, 24, 30, 30, 5, 5, 2, 2),     # 601 columns, strided ragged rows
     # a few k steps in all (not a "same" layer: Winograd's sums, which such small
     # ones take, cancel, and its error has no bound element by element)
     (1, 16, 32, 5, 6, 3, 3, 1, 0),
