@@ -1303,7 +1303,7 @@ bool split_conv_better(const SlabConv& s) {
         const double small = s.W % 2 == 0 ? (double)((s.N * (s.M / 32) + cus - 1) / cus) * (4.5 + 0.225 * s.C)
                                           : (double)((s.N * (s.M / 16) + 2 * cus - 1) / (2 * cus)) * (3.5 + 0.165 * s.C);
         double split;
-        split_tile_for(s.M, px, K, 1, &split);
+        split_tile_for(s.M, px, K, 1, true, &split);
         return split + 7.0 < small;  // (packing the weights, staging the windows)
     }
     return K > 32 && !(taps > 1 && K <= 448 && (((s.M <= 48 || (s.stride == 1 && s.M <= 64)) && px <= 32768) ||

@@ -485,7 +485,7 @@ int split_conv(const SlabConv& s) {
     a.div_kw = make_fastdiv((uint32_t)s.kw);
     a.div_p = make_fastdiv((uint32_t)P);
     a.div_ow = make_fastdiv((uint32_t)s.OW);
-    int tile = split_tile_for(s.M, pixels, g.K, 1);
+    int tile = split_tile_for(s.M, pixels, g.K, 1, true);
     if (tile == S256x256) tile = S128x128;
     const int bm = tile == S128x128 ? 128 : 64, bn = tile == S64x64K || tile == S64x64 ? 64 : 128;
     g.tiles_m = (int)cdiv(s.M, bm);

@@ -390,17 +390,27 @@ namespace {
 //   2048^2 over 64 / 512   128x128 10 / 31    64x128 8.9 / 32    64x64 10 / 35
 //   1024^2 over 64 / 512   64x64K 5.1 / 11.3  64x64 5.2 / 13.6   128x128 7.5 / 21
 // (a 256x128 tile with second accumulators takes 660 us for 4096^3, the
-// 256x256 one 590).
-struct SplitShape {
-    int bm, bn, bk, threads;
+// 256x256 one 590). The two costs of the narrow tiles for dense operands are
+// fitted to 65 ragged and batched products as well, where three 64x64
+// workgroups on a CU cover each other's partial last k step (64x128 / 64x64, us):
+//   32 x 276x128 over 40 8.2 / 7.0    723x1626 over 126 10.2 / 8.7
+//   85 x 74x128 over 393 17.2 / 15.9  687x2393 over 1263 43.2 / 41.3
+//   162 x 315x89 over 80 21.9 / 23.8  1947x1635 over 92 12.5 / 13.5
+// (the choice is 0.9% from the best tile in the mean, 2.2% with the whole
+// grids' costs). Gathered operands keep those: staging a wide tile costs less.
+struct SplitCost {
     double alone, shared, fixed;
 };
+struct SplitShape {
+    int bm, bn, bk, threads;
+    SplitCost dense, gathered;
+};
 const SplitShape kSplitShapes[S_COUNT] = {
-    {256, 256, 16, 512, 4.55, 4.55, 12.5},
-    {128, 128, 32, 512, 1.5, 1.5, 4.5},
-    {64, 128, 32, 256, 0.93, 0.9, 1.6},
-    {64, 64, 64, 512, 0.45, 0.5, 1.9},
-    {64, 64, 32, 256, 0.61, 0.456, 1.25},
+    {256, 256, 16, 512, {4.55, 4.55, 12.5}, {4.55, 4.55, 12.5}},
+    {128, 128, 32, 512, {1.5, 1.5, 4.5}, {1.5, 1.5, 4.5}},
+    {64, 128, 32, 256, {0.93, 0.9, 1.75}, {0.93, 0.9, 1.6}},
+    {64, 64, 64, 512, {0.45, 0.5, 1.9}, {0.45, 0.5, 1.9}},
+    {64, 64, 32, 256, {0.61, 0.4, 1.0}, {0.61, 0.456, 1.25}},
 };
 
 // The split GEMM takes dense products of more than 32 rows and columns whose
@@ -419,16 +429,17 @@ bool split_eligible(const GemmCall& c) {
 }  // namespace
 
 // The tile of the least estimated time for an unsplit product, and that time
-// in us.
-int split_tile_for(int64_t M, int64_t N, int64_t K, int64_t batch, double* time) {
+// in us. `gathered`: a convolution's operand.
+int split_tile_for(int64_t M, int64_t N, int64_t K, int64_t batch, bool gathered, double* time) {
     int best = S64x64;
     double least = 1e30;
     for (int t = 0; t < S_COUNT; ++t) {
         const SplitShape& s = kSplitShapes[t];
+        const SplitCost& cost = gathered ? s.gathered : s.dense;
         const int64_t per_cu = cdiv(cdiv(M, s.bm) * cdiv(N, s.bn) * batch, (int64_t)num_cus());
         const double steps = (double)(cdiv(K, s.bk) * s.bk) / 32.0;
         const double est =
-            (double)per_cu * (steps * (per_cu > 1 ? s.shared : s.alone) + s.fixed);
+            (double)per_cu * (steps * (per_cu > 1 ? cost.shared : cost.alone) + cost.fixed);
         if (est < least) {
             least = est;
             best = t;
@@ -463,7 +474,7 @@ Plan plan_split(const GemmCall& c) {
         const int64_t kps = cdiv(cdiv(K, slices), 32) * 32;
         return Plan{S64x64, (int)cdiv(K, kps), kps, 0};
     }
-    Plan best{split_tile_for(M, N, K, c.batch), 1, K, 0};
+    Plan best{split_tile_for(M, N, K, c.batch, false), 1, K, 0};
     best.k_per_slice = cdiv(K, kSplitShapes[best.tile].bk) * kSplitShapes[best.tile].bk;
     return best;
 }
