@@ -134,8 +134,9 @@ int nrs_gemm_group(const nrs_gemm_desc *descs, int count);
  * turn (each the nrs_gemm_group of its two products, the first adding to dx
  * with beta_x, the others with 1). All products run in one grouped launch
  * and the sums in a second. When an output overlaps another output or an
- * operand, or the products are small enough for the short-GEMM kernel, the
- * closures' sequence runs instead (same results). */
+ * operand, the products are small enough for the short-GEMM kernel, or a size
+ * is past the grouped kernel's 32-bit tile offsets, the closures' sequence
+ * runs instead (same results). */
 int nrs_matmul_shared_lhs_backward(float *dx, float *const *dw, const float *const *g,
                                    const float *x, const float *const *w, int count,
                                    int64_t rows, int64_t inner, int64_t cols, float beta_x,

@@ -39,8 +39,6 @@
 namespace nrs {
 namespace {
 
-int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
 struct ConvSplitArgs {
     GemmArgs g;  // A weights (output gradient), B image; M, N, K, epilogue
     int C, H, W, taps, kw, stride, pad_h, pad_w, OH, OW;

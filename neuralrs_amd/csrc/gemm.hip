@@ -4,6 +4,7 @@
 #include <algorithm>
 
 #include "gemm_kernel.hpp"
+#include "gemm_plan.hpp"
 #include "gemm_skinny.hpp"
 #include "gemm_wsplit.hpp"
 
@@ -100,8 +101,6 @@ KernelFn kernel_for(int tile, int pf, int layout, bool vec4, int amode, int bmod
         default: return nullptr;
     }
 }
-
-int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
@@ -382,101 +381,35 @@ void launch_reduce(GemmArgs p, int slices) {
 
 namespace {
 
-// Tiles of the split GEMM with what a k step of 32 costs a workgroup (us:
-// `alone` on its CU, `shared` with others there) and what it costs besides
-// (filling the pipeline, the epilogue), fitted to whole grids of
-// 1024^2, 2048^2 and 4096^2 over K = 32 .. 512, e.g. (us)
-//   4096^2 over 64 / 512   256x256 24 / 90    128x128 32 / 117   64x128 28 / 134
-//   2048^2 over 64 / 512   128x128 10 / 31    64x128 8.9 / 32    64x64 10 / 35
-//   1024^2 over 64 / 512   64x64K 5.1 / 11.3  64x64 5.2 / 13.6   128x128 7.5 / 21
-// (a 256x128 tile with second accumulators takes 660 us for 4096^3, the
-// 256x256 one 590). The two costs of the narrow tiles for dense operands are
-// fitted to 65 ragged and batched products as well, where three 64x64
-// workgroups on a CU cover each other's partial last k step (64x128 / 64x64, us):
-//   32 x 276x128 over 40 8.2 / 7.0    723x1626 over 126 10.2 / 8.7
-//   85 x 74x128 over 393 17.2 / 15.9  687x2393 over 1263 43.2 / 41.3
-//   162 x 315x89 over 80 21.9 / 23.8  1947x1635 over 92 12.5 / 13.5
-// (the choice is 0.9% from the best tile in the mean, 2.2% with the whole
-// grids' costs). Gathered operands keep those: staging a wide tile costs less.
-struct SplitCost {
-    double alone, shared, fixed;
-};
-struct SplitShape {
-    int bm, bn, bk, threads;
-    SplitCost dense, gathered;
-};
-const SplitShape kSplitShapes[S_COUNT] = {
-    {256, 256, 16, 512, {4.55, 4.55, 12.5}, {4.55, 4.55, 12.5}},
-    {128, 128, 32, 512, {1.5, 1.5, 4.5}, {1.5, 1.5, 4.5}},
-    {64, 128, 32, 256, {0.93, 0.9, 1.75}, {0.93, 0.9, 1.6}},
-    {64, 64, 64, 512, {0.45, 0.5, 1.9}, {0.45, 0.5, 1.9}},
-    {64, 64, 32, 256, {0.61, 0.4, 1.0}, {0.61, 0.456, 1.25}},
-};
+// The sizes of a dense call, as the planner takes them.
+GemmSize size_of(const GemmCall& c) {
+    GemmSize s{c.layout, c.M, c.N, c.K, c.batch, c.sum_row != nullptr};
+    s.split_k = c.allow_split && c.nchw_P == 0;
+    return s;
+}
 
-// The split GEMM takes dense products of more than 32 rows and columns whose
-// rows leave a 32-bit offset over a tile (a row of ones is built for TN). The
-// f32 tiles keep gathered operands, outputs of at most 32 rows or columns
-// (padding would leave the matrix cores nothing to gain) and reductions under
-// a k step into few tiles (1024 x 1024 over 16: 4.4 us against 4.7; with four
-// tiles a CU the split tiles win again, 4096 x 4096 over 16: 23 against 17).
 bool split_eligible(const GemmCall& c) {
-    const int64_t lda = c.layout == NRS_TN ? c.M : c.K, ldb = c.layout == NRS_NT ? c.K : c.N;
-    return c.amode == OP_DENSE && c.bmode == OP_DENSE && c.M > 32 && c.N > 32 && c.K > 0 &&
-           (c.K >= 32 || cdiv(c.M, 64) * cdiv(c.N, 64) * c.batch >= 4 * (int64_t)num_cus()) &&
-           lda < (1 << 21) && ldb < (1 << 21) && (!c.sum_row || c.layout == NRS_TN);
+    return c.amode == OP_DENSE && c.bmode == OP_DENSE && split_takes(size_of(c), num_cus());
 }
-
-}  // namespace
-
-// The tile of the least estimated time for an unsplit product, and that time
-// in us. `gathered`: a convolution's operand.
-int split_tile_for(int64_t M, int64_t N, int64_t K, int64_t batch, bool gathered, double* time) {
-    int best = S64x64;
-    double least = 1e30;
-    for (int t = 0; t < S_COUNT; ++t) {
-        const SplitShape& s = kSplitShapes[t];
-        const SplitCost& cost = gathered ? s.gathered : s.dense;
-        const int64_t per_cu = cdiv(cdiv(M, s.bm) * cdiv(N, s.bn) * batch, (int64_t)num_cus());
-        const double steps = (double)(cdiv(K, s.bk) * s.bk) / 32.0;
-        const double est =
-            (double)per_cu * (steps * (per_cu > 1 ? cost.shared : cost.alone) + cost.fixed);
-        if (est < least) {
-            least = est;
-            best = t;
-        }
-    }
-    if (time) *time = least;
-    return best;
-}
-
-namespace {
 
 // The group kernel takes any dense product the split GEMM's addressing and
 // row of ones allow.
 bool groupable(const GemmCall& c) {
-    const int64_t lda = c.layout == NRS_TN ? c.M : c.K, ldb = c.layout == NRS_NT ? c.K : c.N;
     return c.amode == OP_DENSE && c.bmode == OP_DENSE && c.batch == 1 && c.nchw_P == 0 &&
-           c.partial_buf == nullptr && c.K > 0 && lda < (1 << 21) &&
-           ldb < (1 << 21) && (!c.sum_row || c.layout == NRS_TN);
+           c.partial_buf == nullptr && group_takes(size_of(c));
 }
 
-// Outputs of few 64x64 tiles over a long reduction are split over K as
-// plan_gemm splits them, others take one tile's time.
-Plan plan_split(const GemmCall& c) {
-    const int64_t M = c.M + (c.sum_row ? 1 : 0), N = c.N, K = c.K;
-    const int64_t cus = num_cus();
-    const int64_t t64 = cdiv(M, 64) * cdiv(N, 64) * c.batch;
-    if (c.allow_split && c.nchw_P == 0 && c.batch == 1 && t64 < cus &&
-        (2 * t64 <= cus || K >= 2048) && K >= 256) {
-        const int64_t want = std::min<int64_t>(256, cdiv(3 * cus, t64));
-        const int64_t max_by_k = std::max<int64_t>(1, K / ((t64 >= 16 ? 8 : 2) * 32));
-        const int64_t slices = std::max<int64_t>(1, std::min(want, max_by_k));
-        const int64_t kps = cdiv(cdiv(K, slices), 32) * 32;
-        return Plan{S64x64, (int)cdiv(K, kps), kps, 0};
-    }
-    Plan best{split_tile_for(M, N, K, c.batch, false), 1, K, 0};
-    best.k_per_slice = cdiv(K, kSplitShapes[best.tile].bk) * kSplitShapes[best.tile].bk;
-    return best;
+}  // namespace
+
+int split_tile_for(int64_t M, int64_t N, int64_t K, int64_t batch, bool gathered, double* time) {
+    return cheapest_split_tile(M, N, K, batch, gathered, num_cus(), time);
+}
+
+namespace {
+
+Plan split_plan(const GemmCall& c) {
+    const SplitPlan p = plan_split(size_of(c), num_cus());
+    return Plan{p.tile, p.slices, p.k_per_slice, 0};
 }
 
 // Partials of a split-K launch: the caller's buffer or the library's scratch.
@@ -511,7 +444,7 @@ int gemm_run(const GemmCall& c) {
     const bool vec4 = vec4_loads(c);
     const bool split = split_eligible(c);
 
-    const Plan pl = split ? plan_split(c)
+    const Plan pl = split ? split_plan(c)
                           : plan_gemm(M + (c.sum_row ? 1 : 0), N, K, batch, vec4, dense,
                                       c.allow_split && c.nchw_P == 0);
     TileShape s;
@@ -664,6 +597,7 @@ int launch_group(const GemmCall* calls, const GroupPlan& gp, float* partials, Ge
         const int i = gp.order[oi];
         const GemmCall& c = calls[i];
         const Plan& pl = gp.plans[i];
+        NRS_ARG_CHECK(groupable(c), "gemm group: a product outside the group kernel's limits");
         const int64_t tiles = cdiv(c.M + (c.sum_row ? 1 : 0), s.bm) * cdiv(c.N, s.bn);
         GemmArgs& p = g.prob[next];
         const int rc = make_args(p, c, s, pl);
@@ -850,10 +784,10 @@ int shared_lhs_backward(float* dx, float* const* dw, const float* const* g, cons
         }
     }
     // One group for all products when every pair would run the group kernel
-    // (not the short-GEMM kernel) and no output overlaps another output or an
-    // operand; otherwise the closures' sequence.
+    // (within its addressing, and not the short-GEMM kernel) and no output
+    // overlaps another output or an operand; otherwise the closures' sequence.
     bool fused = count >= 2 && rows > 0 && inner > 0 && cols > 0 && (rows * inner) % 4 == 0 &&
-                 (inner * cols) % 4 == 0 && aligned16(dx);
+                 (inner * cols) % 4 == 0 && aligned16(dx) && shared_lhs_fits(rows, inner, cols);
     for (int i = 0; i < count && fused; ++i)
         for (const GemmCall& c : pair[i])
             fused = fused && vec4_loads(c) && aligned16(c.C);

@@ -4,6 +4,7 @@
 
 #include "buffer_ops.hpp"
 #include "gemm_call.hpp"
+#include "gemm_plan.hpp"
 
 namespace nrs {
 
@@ -35,11 +36,7 @@ struct GemmArgs {
     const float* mask;
 };
 
-
-
-// Tiles of the split GEMM (gemm_split.hpp), and its kernel for a tile and a
-// layout.
-enum SplitTile { S256x256 = 0, S128x128, S64x128, S64x64K, S64x64, S_COUNT };
+// The split GEMM's kernel for a tile (SplitTile) and a layout (gemm_split.hpp).
 using SplitKernel = void (*)(GemmArgs);
 SplitKernel split_kernel(int tile, int layout);
 // Problems of one group launch: the C ABI's groups (NRS_GEMM_GROUP_MAX) and

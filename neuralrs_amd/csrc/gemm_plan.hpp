@@ -1,0 +1,129 @@
+// Which products the split GEMM (gemm_split.hpp) takes, on which tile and in
+// how many K slices. Host only and free of HIP, so that a CPU test can ask.
+#pragma once
+
+#include <algorithm>
+#include <cstdint>
+
+#include "nrs_hip.h"
+
+namespace nrs {
+
+inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Tiles of the split GEMM.
+enum SplitTile { S256x256 = 0, S128x128, S64x128, S64x64K, S64x64, S_COUNT };
+
+// What a k step of 32 costs a workgroup (us:
+// `alone` on its CU, `shared` with others there) and what it costs besides
+// (filling the pipeline, the epilogue), fitted to whole grids of
+// 1024^2, 2048^2 and 4096^2 over K = 32 .. 512, e.g. (us)
+//   4096^2 over 64 / 512   256x256 24 / 90    128x128 32 / 117   64x128 28 / 134
+//   2048^2 over 64 / 512   128x128 10 / 31    64x128 8.9 / 32    64x64 10 / 35
+//   1024^2 over 64 / 512   64x64K 5.1 / 11.3  64x64 5.2 / 13.6   128x128 7.5 / 21
+// (a 256x128 tile with second accumulators takes 660 us for 4096^3, the
+// 256x256 one 590). The two costs of the narrow tiles for dense operands are
+// fitted to 65 ragged and batched products as well, where three 64x64
+// workgroups on a CU cover each other's partial last k step (64x128 / 64x64, us):
+//   32 x 276x128 over 40 8.2 / 7.0    723x1626 over 126 10.2 / 8.7
+//   85 x 74x128 over 393 17.2 / 15.9  687x2393 over 1263 43.2 / 41.3
+//   162 x 315x89 over 80 21.9 / 23.8  1947x1635 over 92 12.5 / 13.5
+// (the choice is 0.9% from the best tile in the mean, 2.2% with the whole
+// grids' costs). Gathered operands keep those: staging a wide tile costs less.
+struct SplitCost {
+    double alone, shared, fixed;
+};
+struct SplitShape {
+    int bm, bn, bk, threads;
+    SplitCost dense, gathered;
+};
+constexpr SplitShape kSplitShapes[S_COUNT] = {
+    {256, 256, 16, 512, {4.55, 4.55, 12.5}, {4.55, 4.55, 12.5}},
+    {128, 128, 32, 512, {1.5, 1.5, 4.5}, {1.5, 1.5, 4.5}},
+    {64, 128, 32, 256, {0.93, 0.9, 1.75}, {0.93, 0.9, 1.6}},
+    {64, 64, 64, 512, {0.45, 0.5, 1.9}, {0.45, 0.5, 1.9}},
+    {64, 64, 32, 256, {0.61, 0.4, 1.0}, {0.61, 0.456, 1.25}},
+};
+
+// A dense product: C[M][N] over K, `batch` of them, with or without a row of
+// sums; `split_k` if it may be split over K.
+struct GemmSize {
+    int layout;
+    int64_t M, N, K, batch;
+    bool sum_row = false, split_k = true;
+    int64_t lda() const { return layout == NRS_TN ? M : K; }
+    int64_t ldb() const { return layout == NRS_NT ? K : N; }
+};
+
+// Whether the 32-bit byte offsets of a staged tile hold (at most 255 rows and a
+// k step), and a row of ones can be built (TN only).
+inline bool split_addressable(const GemmSize& s) {
+    return s.K > 0 && s.lda() < (1 << 21) && s.ldb() < (1 << 21) &&
+           (!s.sum_row || s.layout == NRS_TN);
+}
+
+// The split GEMM takes dense products of more than 32 rows and columns. The f32
+// tiles keep gathered operands, outputs of at most 32 rows or columns
+// (padding would leave the matrix cores nothing to gain) and reductions under
+// a k step into few tiles (1024 x 1024 over 16: 4.4 us against 4.7; with four
+// tiles a CU the split tiles win again, 4096 x 4096 over 16: 23 against 17).
+inline bool split_takes(const GemmSize& s, int cus) {
+    return s.M > 32 && s.N > 32 && split_addressable(s) &&
+           (s.K >= 32 || cdiv(s.M, 64) * cdiv(s.N, 64) * s.batch >= 4 * (int64_t)cus);
+}
+
+// The group kernel (64x64 tiles) takes products of any size it can address.
+inline bool group_takes(const GemmSize& s) { return split_addressable(s); }
+
+// Whether every product of nrs_matmul_shared_lhs_backward fits the group
+// kernel: dx (+)= g . W^T and dW = x^T . g.
+inline bool shared_lhs_fits(int64_t rows, int64_t inner, int64_t cols) {
+    return group_takes(GemmSize{NRS_NT, rows, inner, cols, 1}) &&
+           group_takes(GemmSize{NRS_TN, inner, cols, rows, 1});
+}
+
+// The tile of the least estimated time for an unsplit product, and that time
+// in us. `gathered`: a convolution's operand.
+inline int cheapest_split_tile(int64_t M, int64_t N, int64_t K, int64_t batch, bool gathered,
+                               int cus, double* time = nullptr) {
+    int best = S64x64;
+    double least = 1e30;
+    for (int t = 0; t < S_COUNT; ++t) {
+        const SplitShape& s = kSplitShapes[t];
+        const SplitCost& cost = gathered ? s.gathered : s.dense;
+        const int64_t per_cu = cdiv(cdiv(M, s.bm) * cdiv(N, s.bn) * batch, (int64_t)cus);
+        const double steps = (double)(cdiv(K, s.bk) * s.bk) / 32.0;
+        const double est =
+            (double)per_cu * (steps * (per_cu > 1 ? cost.shared : cost.alone) + cost.fixed);
+        if (est < least) {
+            least = est;
+            best = t;
+        }
+    }
+    if (time) *time = least;
+    return best;
+}
+
+struct SplitPlan {
+    int tile, slices;
+    int64_t k_per_slice;
+};
+
+// Outputs of few 64x64 tiles over a long reduction are split over K, into
+// about three workgroups a CU, others take one tile's time.
+inline SplitPlan plan_split(const GemmSize& s, int cus) {
+    const int64_t M = s.M + (s.sum_row ? 1 : 0), N = s.N, K = s.K;
+    const int64_t t64 = cdiv(M, 64) * cdiv(N, 64) * s.batch;
+    if (s.split_k && s.batch == 1 && t64 < cus && (2 * t64 <= cus || K >= 2048) && K >= 256) {
+        const int64_t want = std::min<int64_t>(256, cdiv(3 * (int64_t)cus, t64));
+        const int64_t max_by_k = std::max<int64_t>(1, K / ((t64 >= 16 ? 8 : 2) * 32));
+        const int64_t slices = std::max<int64_t>(1, std::min(want, max_by_k));
+        const int64_t kps = cdiv(cdiv(K, slices), 32) * 32;
+        return SplitPlan{S64x64, (int)cdiv(K, kps), kps};
+    }
+    const int tile = cheapest_split_tile(M, N, K, s.batch, false, cus);
+    const int bk = kSplitShapes[tile].bk;
+    return SplitPlan{tile, 1, cdiv(K, bk) * bk};
+}
+
+}  // namespace nrs
