@@ -20,13 +20,15 @@
 //
 // The split is exact for every float of magnitude 2^-110 and more (below,
 // x2 may need bits under bf16's smallest denormal) whose x0 is finite. Both
-// exceptions are seen and computed again on the f32 instructions:
-//  * staging keeps the OR of the bits of every x2 that its bf16 form drops.
-//    If any was set and a result of the wave is below 2^-70 in magnitude
-//    (where those bits could matter), or
-//  * a result of the wave is infinite or NaN (an infinite or NaN input, a
-//    value that rounds past bf16's range, or a true overflow),
-// the wave recomputes its block of C from global memory (f32_block).
+// exceptions are seen and computed again on the f32 instructions, 32x32 blocks
+// of C at a time, from global memory (f32_block):
+//  * staging keeps, for every unit, the OR of the bits of its x2s that their
+//    bf16 form drops. How much those bits matter depends on what they would
+//    have met (2^-134 of a row by 2^120 of a column is a normal result), so
+//    the results of every row of A and column of B that dropped any are
+//    replaced, whatever their size;
+//  * a block with a result that is infinite or NaN (an infinite or NaN input,
+//    a value that rounds past bf16's range, or a true overflow) is replaced.
 //
 // A workgroup of WAVES_M x WAVES_N waves owns a BM x BN block of C. Operand
 // tiles of BK k values are loaded to registers one k-tile ahead, split, and
@@ -236,40 +238,24 @@ struct SplitOperand {
     }
 };
 
-// The wave's (32 FM) x (32 FN) block at (m0, n0) of the tile over [kbeg, kend)
-// on the f32 instructions, operands element by element from global memory (the
-// exceptions above: any inputs, no staging, not fast).
-template <int FM, int FN, class OA, class OB>
-__device__ __forceinline__ void f32_block(f32x16 (&acc)[FM][FN], const OA& oa, const OB& ob, int m0,
-                                          int n0, int64_t kbeg, int64_t kend, int lane) {
+// The 32 x 32 block at (m0, n0) of the tile over [kbeg, kend) on the f32
+// instructions, operands element by element from global memory (the exceptions
+// above: any inputs, no staging, not fast).
+template <class OA, class OB>
+__device__ __forceinline__ f32x16 f32_block(const OA& oa, const OB& ob, int m0, int n0, int64_t kbeg,
+                                            int64_t kend, int lane) {
     const int h = lane >> 5, l32 = lane & 31;
+    f32x16 acc;
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
 #pragma unroll 1
     for (int64_t k = kbeg; k < kend; k += 2) {
         const bool ok = k + h < kend;
         const int64_t kk = ok ? k + h : kbeg;
-        float a[FM], b[FN];
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            const float x = oa.at(m0 + 32 * i + l32, kk);
-            a[i] = ok ? x : 0.0f;
-        }
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            const float x = ob.at(n0 + 32 * j + l32, kk);
-            b[j] = ok ? x : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+        const float x = oa.at(m0 + l32, kk), y = ob.at(n0 + l32, kk);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ok ? x : 0.0f, ok ? y : 0.0f, acc, 0, 0, 0);
     }
+    return acc;
 }
 
 // The tile at (m0, n0) over [kbeg, kend) of the product of the initialised
@@ -297,7 +283,6 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
                 acc[i][j][r] = 0.0f;
                 if constexpr (TWO) lo[i][j][r] = 0.0f;
             }
-    uint32_t sticky = 0;
     f32x4 ra[C_::UA][2], rb[C_::UB][2];
 
     const int ntiles = (int)((kend - kbeg + BK - 1) / BK);
@@ -306,6 +291,9 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
     constexpr bool kMasked = OA::kMasked && OB::kMasked;
     const int nfull = kMasked ? ntiles : (int)((kend - kbeg) / BK);
     constexpr int kUnits = C_::UA + C_::UB;
+    uint32_t sticky[kUnits];
+#pragma unroll
+    for (int un = 0; un < kUnits; ++un) sticky[un] = 0;
     auto load_unit = [&](int t, int un, auto part) {
         constexpr bool PART = decltype(part)::value;
         const int64_t k0 = kbeg + (int64_t)t * BK;
@@ -338,7 +326,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
         constexpr bool in_a = un < C_::UA;
         constexpr int i = in_a ? un : un - C_::UA;
         if constexpr (!in_a && OB::kFix && x % kSplitSteps == 0) ob.fix(rb[i], i);
-        st.template step<x % kSplitSteps>(in_a ? ra[i] : rb[i], sticky,
+        st.template step<x % kSplitSteps>(in_a ? ra[i] : rb[i], sticky[un],
                                           in_a ? OA::kOnes && ((oa.ones >> i) & 1u)
                                                : OB::kOnes && ((ob.ones >> i) & 1u));
         if constexpr (x % kSplitSteps == kSplitSteps - 1) {
@@ -456,17 +444,40 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
 #pragma unroll
             for (int j = 0; j < FN; ++j) acc[i][j] = acc[i][j] + lo[i][j];
     }
-    const int lost = __syncthreads_or((int)(sticky & 0xffffu));
+    uint32_t dropped = 0;
+#pragma unroll
+    for (int un = 0; un < kUnits; ++un) dropped |= sticky[un];
+    const bool lost = __syncthreads_or((int)(dropped & 0xffffu));
+    // (the barrier above: every wave is done with the staging buffers)
+    // A bit for each row and column of the tile with dropped bits, past what
+    // the wave sets exchange.
+    constexpr int kFlags = (BM + BN) / 32;
+    uint32_t* const flags = reinterpret_cast<uint32_t*>(smem + 2 * C_::STAGE) - kFlags;
+    if (lost) {  // uniform
+        if (tid < kFlags) flags[tid] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int un = 0; un < kUnits; ++un) {
+            int row, q;
+            if (un < C_::UA)
+                split_pos<BM, BK, OA::kKC, NT>(un, tid, row, q);
+            else
+                split_pos<BN, BK, OB::kKC, NT>(un - C_::UA, tid, row, q);
+            if (un >= C_::UA) row += BM;
+            if (sticky[un] & 0xffffu) atomicOr(flags + row / 32, 1u << (row % 32));
+        }
+        __syncthreads();
+    }
     if constexpr (KS == 1) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int j = 0; j < FN; ++j) out[i][j] = acc[i][j];
     } else {
-        // (the barrier above: every wave is done with the staging buffers)
         float* x = reinterpret_cast<float*>(smem);
         constexpr int WS = WAVES_M * WAVES_N, BLK = FM * FO * 1024;
-        static_assert((kShare ? 2 : 1) * WS * BLK * 4 <= 2 * C_::STAGE * 16, "k-split LDS space");
+        static_assert((kShare ? 2 : 1) * WS * BLK * 4 + kFlags * 4 <= 2 * C_::STAGE * 16,
+                      "k-split LDS space");
         if (kShare || kset == 1) {
 #pragma unroll
             for (int i = 0; i < FM; ++i)
@@ -496,26 +507,29 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
                 }
     }
 
-    // The exceptions: dropped bits of some x2 in the workgroup's operands
-    // beside small results, or a result that is not finite.
-    float finite = 0.0f;  // 0 while every result is finite, else NaN
-    bool small = false;
+    // The exceptions: rows and columns with dropped bits, and blocks with a
+    // result that is not finite.
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FO; ++j)
+        for (int j = 0; j < FO; ++j) {
+            float finite = 0.0f;  // 0 while every result is finite, else NaN
 #pragma unroll
             for (int r = 0; r < 16; ++r) finite = fmaf(out[i][j][r], 0.0f, finite);
-    if (lost) {  // uniform
+            const bool all = __any(finite != 0.0f);
+            uint32_t rows = 0, cols = 0;
+            if (lost) {  // uniform
+                rows = flags[wm0 / 32 + i];
+                cols = flags[(BM + wo0) / 32 + j];
+            }
+            if (all || rows || cols) {  // uniform
+                const f32x16 f = f32_block(oa, ob, wm0 + 32 * i, wo0 + 32 * j, kbeg, kend, lane);
+                const bool col = all || ((cols >> l32) & 1u);
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FO; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) small |= fabsf(out[i][j][r]) < 0x1p-70f;
-    }
-    if (__any(small || finite != 0.0f))
-        f32_block<FM, FO>(out, oa, ob, wm0, wo0, kbeg, kend, lane);
+                for (int r = 0; r < 16; ++r)
+                    if (col || ((rows >> (8 * (r / 4) + 4 * h + r % 4)) & 1u)) out[i][j][r] = f[r];
+            }
+        }
 
     const TileOut<FO> to = tile_out<BM, BN, FO>(p, m0, n0, wm0, wo0, h, l32, slice, batch);
     const float none[1][1][16] = {};

@@ -143,3 +143,23 @@ def test_infinities_and_nan_stay_where_they_belong(hip, shape):
         assert not np.isfinite(got[k][bad]).any()
         ok = ~bad
         assert np.all(np.abs(got[k][ok] - f[ok]) <= 1e-4 * np.abs(f[ok]) + 1e-30)
+
+
+@pytest.mark.parametrize("tiny", range(3))
+@pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[1], SHAPES[3], SHAPES[8], SHAPES[11], SHAPES[15]], ids=IDS)
+def test_tiny_times_huge(hip, shape, tiny):
+    """One of image, weights and gradient below the split's exact range, the
+    others large: the bits it drops would show in results of any size."""
+    sx, sw, sb, sg = sizes(shape)
+    rng = np.random.default_rng(7 + sum(shape) + tiny)
+    make = lambda s, e: np.ldexp(rng.random(s) + 0.5, e).astype(np.float32)
+    x, w, g = (make(s, -118 if i == tiny else 54) for i, s in enumerate((sx, sw, sg)))
+    b = np.zeros(sb, np.float32)
+    nan = [np.full(s, np.nan, np.float32) for s in (sx, sw, sb)]
+    got = run(hip, shape, x, w, b, g, nan, 0.0, 0.0)
+    want, size = reference(shape, x, w, b, g), reference(shape, *map(np.abs, (x, w, b, g)))
+    ks = (sw[1] * sw[2] * sw[3], sw[0] * sw[2] * sw[3], sg[0] * sg[2] * sg[3], sg[0] * sg[2] * sg[3])
+    for k, name in enumerate(("output", "input gradient", "weight gradient", "bias gradient")):
+        # (f32 instructions round every product and sum)
+        bound = (ks[k] + 72) * 2.0 ** -24 * size[k]
+        assert np.all(np.abs(got[k] - want[k]) <= bound), name

@@ -158,6 +158,49 @@ def test_tiny_magnitudes(hip, layout, shape):
     assert np.all(np.abs(got - A[sample] @ B) <= bound)
 
 
+# exponents of the tiny and the huge operand: the tiny one's third piece is
+# dropped in part, the second one too, and almost all of it
+@pytest.mark.parametrize("tiny,huge", [(-118, 62), (-127, 98), (-134, 108)])
+@pytest.mark.parametrize("layout", [NN, NT, TN])
+@pytest.mark.parametrize("shape", [(129, 200, 70), (1000, 1333, 65), (4096, 256, 130), (64, 576, 5000),
+                                   (4096, 4096, 48)], ids=IDS)
+def test_tiny_times_huge(hip, layout, shape, tiny, huge):
+    """Bits that the split of a tiny operand drops matter as much as the other
+    operand makes them, with results of any size."""
+    rows, cols, inner = shape
+    rng = np.random.default_rng(11 * rows + layout - tiny)
+    small = lambda s: np.ldexp(rng.standard_normal(s), tiny).astype(np.float32)
+    large = lambda s: np.ldexp(rng.standard_normal(s), huge).astype(np.float32)
+    sample = np.unique(np.linspace(0, rows - 1, 97).astype(int))
+    for ma, mb in ((small, large), (large, small)):
+        a, b = operands(layout, rows, cols, inner, ma, mb)
+        A, B = logical(layout, a, b)
+        got = gemm(hip, layout, a, b, rows, cols, inner)[sample]
+        # (f32 instructions round every product and sum)
+        bound = (inner + 8) * 2.0 ** -24 * (np.abs(A[sample]) @ np.abs(B))
+        assert np.all(np.abs(got - A[sample] @ B) <= bound)
+
+
+def test_tiny_times_huge_in_a_group(hip):
+    """The products of a Linear's backward, which share one launch: a single
+    tiny value of a row that is otherwise zero, and of a column."""
+    rng = np.random.default_rng(3)
+    batch, in_f, out_f = 4096, 128, 192
+    x = rng.standard_normal((batch, in_f)).astype(np.float32)
+    w = np.ldexp(rng.standard_normal((in_f, out_f)), 90).astype(np.float32)
+    g = np.zeros((batch, out_f), np.float32)
+    g[5, 7], g[77, 100], g[4000] = 1.2345678e-36, 2.0 ** -129 * 1.37, np.float32(1.2345678e-38)
+    x[5] *= np.float32(2.0 ** 80)
+    dx, dw = hip.DeviceBuffer(batch * in_f), hip.DeviceBuffer(in_f * out_f)
+    hip.call("nrs_linear_backward", dx, dw, None, hip.DeviceBuffer.from_host(g),
+             hip.DeviceBuffer.from_host(x), hip.DeviceBuffer.from_host(w), batch, in_f, out_f, 0.0, 0.0, 0.0)
+    X, W, G = (v.astype(np.float64) for v in (x, w, g))
+    for got, want, size, k in ((dx.to_host((batch, in_f)), G @ W.T, np.abs(G) @ np.abs(W.T), out_f),
+                               (dw.to_host((in_f, out_f)), X.T @ G, np.abs(X.T) @ np.abs(G), batch)):
+        # (2^-149: results under f32's smallest normal value)
+        assert np.all(np.abs(got - want) <= (k + 8) * 2.0 ** -24 * size + k * 2.0 ** -149)
+
+
 def test_bmm_large_items(hip):
     """Batched items past the small-item kernel, each at its own offset."""
     rng = np.random.default_rng(1)
