@@ -146,15 +146,27 @@ struct ConvPixels {
                     float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, voff, s0 + e * plane4, 0));
         }
     }
-    __device__ __forceinline__ float at(int col, int64_t k) const {
+    struct Spot {
+        int off, iy0, ix0;  // bytes of the pixel's window corner, and where it lies
+    };
+    __device__ __forceinline__ Spot spot(int col) const {
         int img, iy0, ix0;
         corner(n0 + col, img, iy0, ix0);
+        return Spot{(img * a->C * a->H * a->W + (iy0 + a->pad_h) * a->W + ix0 + a->pad_w) * 4, iy0, ix0};
+    }
+    template <bool PART>  // (K is a multiple of 4: a quad ends before it or begins past it)
+    __device__ __forceinline__ void four(f32x4& x, const Spot& s, int64_t k, int dk, int64_t kend) const {
+        const auto rsrc = buffer_rsrc(base, 0x80000000ll);
+        const int plane4 = a->H * a->W * 4;
         uint32_t tap, c, ti, tj;
-        fast_divmod((uint32_t)k, a->div_c, tap, c);
+        fast_divmod((uint32_t)k + dk, a->div_c, tap, c);
         fast_divmod(tap, a->div_kw, ti, tj);
-        const int y = iy0 + (int)ti, x = ix0 + (int)tj;
-        if ((unsigned)y >= (unsigned)a->H || (unsigned)x >= (unsigned)a->W) return 0.0f;
-        return a->g.B[(((int64_t)img * a->C + c) * a->H + y) * a->W + x];
+        const bool in = ((unsigned)(s.iy0 + (int)ti) < (unsigned)a->H) &
+                        ((unsigned)(s.ix0 + (int)tj) < (unsigned)a->W) & (!PART || k + dk < kend);
+        const int at = in ? s.off + (int)c * plane4 + ((int)ti * a->W + (int)tj) * 4 : kOutOfRange;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            x[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at, e * plane4, 0));
     }
 };
 
@@ -189,31 +201,35 @@ ConvKernel conv_kernel(int tile, int channels) {
 
 // ------------------------------------------------------------ weight gradient
 
-// The two quads of output pixels that a thread's units of a k-tile cover.
-struct QuadPos {
-    int live[2];         // pixels of the quad inside its row (0: past the end)
-    int g_off[2];        // bytes of the quad in a channel plane of the gradient
-    int x_off[2];        // bytes of its window corner in the image's first plane
-    int iy0[2], ix0[2];  // that corner
-};
+// The quad of output pixels at k.
+struct QuadAt {
+    int live;      // pixels of the quad inside its row (0: past the end)
+    int g_off;     // bytes of the quad in a channel plane of the gradient
+    int x_off;     // bytes of its window corner in the image's first plane
+    int iy0, ix0;  // that corner
 
-template <int BK>
-__device__ __forceinline__ void quad_pos(QuadPos& p, const ConvSplitArgs& a, int64_t k0, int tid) {
-    const int q = tid % (BK / 8);
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        const int quad = (int)(k0 >> 2) + half * (BK / 8) + q;
+    QuadAt() = default;
+    __device__ __forceinline__ QuadAt(const ConvSplitArgs& a, int k) {
+        const int quad = k >> 2;
         const bool in = quad < a.quads;
         uint32_t row, qx, img, oy;
         fast_divmod((uint32_t)(in ? quad : 0), a.div_rowq, row, qx);
         fast_divmod(row, a.div_oh, img, oy);
         const int ox = 4 * (int)qx;
-        p.live[half] = in ? a.OW - ox : 0;
-        p.g_off[half] = ((int)img * (int)a.g.M * a.OH * a.OW + (int)oy * a.OW + ox) * 4;
-        p.iy0[half] = (int)oy * a.stride - a.pad_h;
-        p.ix0[half] = ox * a.stride - a.pad_w;
-        p.x_off[half] = ((int)img * a.C * a.H * a.W + (int)oy * a.stride * a.W + ox * a.stride) * 4;
+        live = in ? a.OW - ox : 0;
+        g_off = ((int)img * (int)a.g.M * a.OH * a.OW + (int)oy * a.OW + ox) * 4;
+        iy0 = (int)oy * a.stride - a.pad_h;
+        ix0 = ox * a.stride - a.pad_w;
+        x_off = ((int)img * a.C * a.H * a.W + (int)oy * a.stride * a.W + ox * a.stride) * 4;
     }
+};
+
+// The two quads that a thread's units of a k-tile cover.
+template <int BK>
+__device__ __forceinline__ void quad_pos(QuadAt (&p)[2], const ConvSplitArgs& a, int64_t k0, int tid) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+        p[half] = QuadAt(a, (int)k0 + half * (BK / 2) + 4 * (tid % (BK / 8)));
 }
 
 // The output gradient [channel][pixel]. QUADS: rows are whole quads.
@@ -222,14 +238,14 @@ struct GradRows {
     static constexpr bool kKC = true, kOnes = false, kMasked = true, kFix = false;
     static constexpr uint32_t ones = 0;
     const ConvSplitArgs* a;
-    const QuadPos* pos;
+    const QuadAt* pos;  // [2]
     int64_t m0;
     int off[U];
 
-    __device__ __forceinline__ void init(const ConvSplitArgs& args, const QuadPos& p, int64_t m0_,
+    __device__ __forceinline__ void init(const ConvSplitArgs& args, const QuadAt* p, int64_t m0_,
                                          int tid) {
         a = &args;
-        pos = &p;
+        pos = p;
         m0 = m0_;
 #pragma unroll
         for (int i = 0; i < U; ++i) {
@@ -240,30 +256,29 @@ struct GradRows {
     }
     __device__ __forceinline__ void begin(int64_t, int) {}
     __device__ __forceinline__ void fix(f32x4 (&)[2], int) const {}
-    template <bool PART>
-    __device__ __forceinline__ void load(f32x4 (&r)[2], int i, int64_t, int64_t, int) const {
+    // The quad p of the channel at `off`.
+    __device__ __forceinline__ void fetch(f32x4& r, int off, const QuadAt& p) const {
         const auto rsrc = buffer_rsrc(a->g.A, 0x80000000ll);
+        const int at = off + p.g_off;
+        if constexpr (QUADS) {
+            r = buffer_load4(rsrc, p.live > 0 ? at : kOutOfRange);
+        } else {
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const int at = off[i] + pos->g_off[half];
-            if constexpr (QUADS) {
-                r[half] = buffer_load4(rsrc, pos->live[half] > 0 ? at : kOutOfRange);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    r[half][e] = buffer_load1(rsrc, e < pos->live[half] ? at + 4 * e : kOutOfRange);
-            }
+            for (int e = 0; e < 4; ++e) r[e] = buffer_load1(rsrc, e < p.live ? at + 4 * e : kOutOfRange);
         }
     }
-    __device__ __forceinline__ float at(int row, int64_t k) const {
-        uint32_t rw, qx, img, oy;
-        if ((k >> 2) >= a->quads) return 0.0f;
-        fast_divmod((uint32_t)(k >> 2), a->div_rowq, rw, qx);
-        fast_divmod(rw, a->div_oh, img, oy);
-        const int ox = 4 * (int)qx + (int)(k & 3);
-        if (ox >= a->OW) return 0.0f;
-        const int64_t m = min(m0 + row, a->g.M - 1);
-        return a->g.A[(((int64_t)img * a->g.M + m) * a->OH + oy) * a->OW + ox];
+    template <bool PART>
+    __device__ __forceinline__ void load(f32x4 (&r)[2], int i, int64_t, int64_t, int) const {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) fetch(r[half], off[i], pos[half]);
+    }
+    using Spot = int;  // bytes of the row's channel in an image
+    __device__ __forceinline__ Spot spot(int row) const {
+        return (int)min(m0 + row, a->g.M - 1) * a->OH * a->OW * 4;
+    }
+    template <bool PART>  // (slices are whole k steps, the last one masked by the quads)
+    __device__ __forceinline__ void four(f32x4& x, const Spot& s, int64_t k, int dk, int64_t) const {
+        fetch(x, s, QuadAt(*a, (int)k + dk));
     }
 };
 
@@ -271,12 +286,12 @@ struct GradRows {
 // NEAR: whole quads of a stride-1 layer with at most one column of padding: a
 // quad's four window pixels are one 128-bit load (a quarter of the load
 // instructions). Where the window's first or last pixel is outside the image
-// the load moves one pixel in, and `fix` moves the values back.
+// the load moves one pixel in, and `settle` moves the values back.
 template <int BN, int BK, int NT, int U, bool NEAR>
 struct WindowRows {
     static constexpr bool kKC = true, kOnes = true, kMasked = true, kFix = NEAR;
     const ConvSplitArgs* a;
-    QuadPos pos;
+    QuadAt pos[2];
     const float* base;  // the image, one padding corner before its start
     int64_t n0;
     int off[U], ti[U], tj[U];
@@ -302,58 +317,62 @@ struct WindowRows {
         }
     }
     __device__ __forceinline__ void begin(int64_t k0, int tid) { quad_pos<BK>(pos, *a, k0, tid); }
-    template <bool PART>
-    __device__ __forceinline__ void load(f32x4 (&r)[2], int i, int64_t, int64_t, int) {
+    // The window pixels of quad p at tap (ty, tx), `off` bytes from its corner;
+    // returns what `settle` has to know.
+    __device__ __forceinline__ uint32_t fetch(f32x4& r, int off, int ty, int tx, const QuadAt& p) const {
         const auto rsrc = buffer_rsrc(base, 0x80000000ll);
+        const bool row_in = (unsigned)(p.iy0 + ty) < (unsigned)a->H;
         if constexpr (NEAR) {
-            moved[i] = 0;
-#pragma unroll
-            for (int half = 0; half < 2; ++half) {
-                const int ix = pos.ix0[half] + tj[i];
-                const bool in = ((unsigned)(pos.iy0[half] + ti[i]) < (unsigned)a->H) & (pos.live[half] > 0);
-                const bool left = ix < 0, right = ix + 3 >= a->W;
-                const int at = off[i] + pos.x_off[half] + (left ? 4 : 0) - (right ? 4 : 0);
-                moved[i] |= ((uint32_t)left | (uint32_t)right << 1) << (2 * half);
-                r[half] = buffer_load4(rsrc, in ? at : kOutOfRange);
-            }
-            return;
-        }
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const int at = off[i] + pos.x_off[half];
-            const bool row_in = (unsigned)(pos.iy0[half] + ti[i]) < (unsigned)a->H;
-            const int ix = row_in ? pos.ix0[half] + tj[i] : -(1 << 28);
+            const int ix = p.ix0 + tx;
+            const bool in = row_in & (p.live > 0);
+            const bool left = ix < 0, right = ix + 3 >= a->W;
+            const int at = off + p.x_off + (left ? 4 : 0) - (right ? 4 : 0);
+            r = buffer_load4(rsrc, in ? at : kOutOfRange);
+            return (uint32_t)left | (uint32_t)right << 1;
+        } else {
+            const int at = off + p.x_off, ix = row_in ? p.ix0 + tx : -(1 << 28);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const bool ok = ((unsigned)(ix + e * a->stride) < (unsigned)a->W) & (e < pos.live[half]);
-                r[half][e] = buffer_load1(rsrc, ok ? at + 4 * e * a->stride : kOutOfRange);
+                const bool ok = ((unsigned)(ix + e * a->stride) < (unsigned)a->W) & (e < p.live);
+                r[e] = buffer_load1(rsrc, ok ? at + 4 * e * a->stride : kOutOfRange);
             }
+            return 0;
         }
+    }
+    static __device__ __forceinline__ void settle(f32x4& r, uint32_t moved) {
+        if constexpr (NEAR) {
+            const bool left = moved & 1u, right = moved & 2u;
+            const f32x4 v = r;
+            r = f32x4{right ? v[1] : (left ? 0.0f : v[0]), right ? v[2] : (left ? v[0] : v[1]),
+                      right ? v[3] : (left ? v[1] : v[2]), right ? 0.0f : (left ? v[2] : v[3])};
+        }
+    }
+    template <bool PART>
+    __device__ __forceinline__ void load(f32x4 (&r)[2], int i, int64_t, int64_t, int) {
+        moved[i] = 0;
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+            moved[i] |= fetch(r[half], off[i], ti[i], tj[i], pos[half]) << (2 * half);
     }
     __device__ __forceinline__ void fix(f32x4 (&r)[2], int i) const {
-        if constexpr (NEAR) {
 #pragma unroll
-            for (int half = 0; half < 2; ++half) {
-                const bool left = (moved[i] >> (2 * half)) & 1u, right = (moved[i] >> (2 * half)) & 2u;
-                const f32x4 v = r[half];
-                r[half] = f32x4{right ? v[1] : (left ? 0.0f : v[0]), right ? v[2] : (left ? v[0] : v[1]),
-                                right ? v[3] : (left ? v[1] : v[2]), right ? 0.0f : (left ? v[2] : v[3])};
-            }
-        }
+        for (int half = 0; half < 2; ++half) settle(r[half], moved[i] >> (2 * half));
     }
-    __device__ __forceinline__ float at(int col, int64_t k) const {
-        if (n0 + col >= columns()) return n0 + col == columns() ? 1.0f : 0.0f;
-        uint32_t c, tap, ty, tx, rw, qx, img, oy;
-        if ((k >> 2) >= a->quads) return 0.0f;
-        fast_divmod((uint32_t)(n0 + col), a->div_taps, c, tap);
+    struct Spot {
+        int off, ty, tx;  // bytes of the channel's tap in an image, and the tap
+        bool ones;
+    };
+    __device__ __forceinline__ Spot spot(int col) const {  // (columns past the ones are not stored)
+        uint32_t c, tap, ty, tx;
+        fast_divmod((uint32_t)min(n0 + col, columns() - 1), a->div_taps, c, tap);
         fast_divmod(tap, a->div_kw, ty, tx);
-        fast_divmod((uint32_t)(k >> 2), a->div_rowq, rw, qx);
-        fast_divmod(rw, a->div_oh, img, oy);
-        const int ox = 4 * (int)qx + (int)(k & 3);
-        const int y = (int)oy * a->stride - a->pad_h + (int)ty;
-        const int x = ox * a->stride - a->pad_w + (int)tx;
-        if (ox >= a->OW || (unsigned)y >= (unsigned)a->H || (unsigned)x >= (unsigned)a->W) return 0.0f;
-        return a->g.B[(((int64_t)img * a->C + c) * a->H + y) * a->W + x];
+        return Spot{((int)c * a->H * a->W + (int)ty * a->W + (int)tx) * 4, (int)ty, (int)tx,
+                    n0 + col == columns()};
+    }
+    template <bool PART>
+    __device__ __forceinline__ void four(f32x4& x, const Spot& s, int64_t k, int dk, int64_t) const {
+        settle(x, fetch(x, s.off, s.ty, s.tx, QuadAt(*a, (int)k + dk)));
+        if (s.ones) x = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
     }
 };
 

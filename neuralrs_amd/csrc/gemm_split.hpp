@@ -164,8 +164,9 @@ __device__ __forceinline__ void split_pos(int i, int tid, int& row, int& q) {
 // (What split_tile asks of an operand: kKC, the order of its units over the
 // threads; kOnes and `ones`, bit i set where unit i is all ones; kMasked, true
 // if load<false> reads zero past the end of k; begin, called before the first
-// unit of a k-tile is loaded; load; at, any one element; and kFix, of a column
-// operand whose loaded units go through fix before they are split.)
+// unit of a k-tile is loaded; load; spot and four, a row and 4 k values of it
+// as f32_block takes them, k a multiple of 4; and kFix, of a column operand whose
+// loaded units go through fix before they are split.)
 template <int BMN, int BK, bool KC, int NT, int U, bool ONES = false>
 struct SplitOperand {
     static constexpr bool kKC = KC, kOnes = ONES, kMasked = false, kFix = false;
@@ -197,10 +198,46 @@ struct SplitOperand {
     __device__ __forceinline__ void begin(int64_t, int) {}
     __device__ __forceinline__ void fix(f32x4 (&)[2], int) const {}
 
-    __device__ __forceinline__ float at(int row, int64_t k) const {
+    struct Spot {
+        int off;  // bytes of the row at k = 0 of the tile
+        bool one;
+    };
+    __device__ __forceinline__ Spot spot(int row) const {
         const int r = min(row, last);
-        const float x = KC ? base[r * ld + k] : base[k * ld + r];
-        return ONES && row == one_row ? 1.0f : x;
+        return Spot{4 * (KC ? r * (int)ld : r), ONES && row == one_row};
+    }
+    // Elements k + dk .. k + dk + 3 of a row, k uniform; with PART, zero at or
+    // past kend.
+    template <bool PART>
+    __device__ __forceinline__ void four(f32x4& x, const Spot& s, int64_t k, int dk, int64_t kend) const {
+        const auto rsrc = at_k(k);
+        const int off = s.off + 4 * dk * (KC ? 1 : (int)ld);
+        if constexpr (KC && !PART) {
+            x = buffer_load4(rsrc, off);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int soff = 4 * e * (KC ? 1 : (int)ld);
+                if constexpr (PART)
+                    x[e] = buffer_load1(rsrc, k + dk + e < kend ? off + soff : kOutOfRange);
+                else
+                    x[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, off, soff, 0));
+            }
+        }
+        if constexpr (ONES) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = s.one ? (PART && k + dk + e >= kend ? 0.0f : 1.0f) : x[e];
+        }
+    }
+
+    // The operand from k on. (Kept scalar: the compiler may hold a uniform loop
+    // value in vector registers, and would then loop over the lanes of every
+    // load.)
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t at_k(int64_t k) const {
+        const uint64_t at = (uint64_t)(base + (KC ? k : k * ld));
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)at);
+        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));
+        return buffer_rsrc((const float*)((uint64_t)hi << 32 | lo), 0x80000000ll);
     }
 
     // Loads unit i of the k-tile at k0. PART: elements at or past kend read
@@ -210,12 +247,7 @@ struct SplitOperand {
                                          int tid) const {
         int row, q;
         split_pos<BMN, BK, KC, NT>(i, tid, row, q);
-        // (kept scalar: the compiler may hold a uniform loop value in vector
-        // registers, and would then loop over the lanes of every load)
-        const uint64_t at = (uint64_t)(base + (KC ? k0 : k0 * ld));
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)at);
-        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));
-        const auto rsrc = buffer_rsrc((const float*)((uint64_t)hi << 32 | lo), 0x80000000ll);
+        const auto rsrc = at_k(k0);
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
             const int kk = half * (BK / 2);  // k of the unit's half, less 4q
@@ -239,21 +271,62 @@ struct SplitOperand {
 };
 
 // The 32 x 32 block at (m0, n0) of the tile over [kbeg, kend) on the f32
-// instructions, operands element by element from global memory (the exceptions
-// above: any inputs, no staging, not fast).
+// instructions, operands from global memory (the exceptions above: any inputs,
+// no staging). A step takes 16 k values, 8 of each operand a lane; the next two
+// steps' loads are in flight meanwhile. It is bound by the latency of those
+// loads where a few blocks are redone, by the L1 lines they touch where all
+// are. Time of a call, us, with ordinary inputs / one row of NaN / NaN
+// throughout (the values one by one, a step ahead: in brackets):
+//   NN 4096^3              600 / 773 / 1715   (1868, 5857)
+//   NT 1000 x 1333 x 777    26 / 47 / 51      (103, 138)
+//   TN 2048 x 2048 x 512    28 / 55 / 80      (101, 131)
+//   NT 64 x 576 x 100352    66 / 121 / 156    (279, 465)
+//   64->128 3x3 32 x 32^2   41 / 92 / 89 and 49 / 117 / 116   (234, 336)
+// Inputs that drop bits in one row or throughout cost the same.
 template <class OA, class OB>
 __device__ __forceinline__ f32x16 f32_block(const OA& oa, const OB& ob, int m0, int n0, int64_t kbeg,
                                             int64_t kend, int lane) {
     const int h = lane >> 5, l32 = lane & 31;
+    const auto sa = oa.spot(m0 + l32);
+    const auto sb = ob.spot(n0 + l32);
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    constexpr int kAhead = 3;  // steps in registers
+    f32x4 x[kAhead][2], y[kAhead][2];
+    auto load = [&](f32x4(&a)[2], f32x4(&b)[2], int step, auto part) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            oa.template four<decltype(part)::value>(a[u], sa, kbeg + 16 * step, 8 * h + 4 * u, kend);
+            ob.template four<decltype(part)::value>(b[u], sb, kbeg + 16 * step, 8 * h + 4 * u, kend);
+        }
+    };
+    auto multiply = [&](const f32x4(&a)[2], const f32x4(&b)[2]) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][e], b[u][e], acc, 0, 0, 0);
+    };
+    constexpr std::integral_constant<bool, true> yes{};
+    constexpr std::integral_constant<bool, false> no{};
+    const int full = (int)((kend - kbeg) / 16);
+    if (full > 0) {  // (the last whole step again, unused, past the end)
+#pragma unroll
+        for (int u = 0; u < kAhead - 1; ++u) load(x[u], y[u], min(u, full - 1), no);
+    }
 #pragma unroll 1
-    for (int64_t k = kbeg; k < kend; k += 2) {
-        const bool ok = k + h < kend;
-        const int64_t kk = ok ? k + h : kbeg;
-        const float x = oa.at(m0 + l32, kk), y = ob.at(n0 + l32, kk);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ok ? x : 0.0f, ok ? y : 0.0f, acc, 0, 0, 0);
+    for (int t = 0; t < full; t += kAhead) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            constexpr int d = kAhead - 1;
+            load(x[(u + d) % kAhead], y[(u + d) % kAhead], min(t + u + d, full - 1), no);
+            if (t + u < full) multiply(x[u], y[u]);  // uniform
+        }
+    }
+    if (kbeg + 16 * (int64_t)full < kend) {
+        load(x[0], y[0], full, yes);
+        multiply(x[0], y[0]);
     }
     return acc;
 }
@@ -508,7 +581,8 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
     }
 
     // The exceptions: rows and columns with dropped bits, and blocks with a
-    // result that is not finite.
+    // result that is not finite (bit i * FO + j of `redo` and `all`).
+    uint32_t redo = 0, all = 0;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -516,20 +590,28 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
             float finite = 0.0f;  // 0 while every result is finite, else NaN
 #pragma unroll
             for (int r = 0; r < 16; ++r) finite = fmaf(out[i][j][r], 0.0f, finite);
-            const bool all = __any(finite != 0.0f);
-            uint32_t rows = 0, cols = 0;
-            if (lost) {  // uniform
-                rows = flags[wm0 / 32 + i];
-                cols = flags[(BM + wo0) / 32 + j];
-            }
-            if (all || rows || cols) {  // uniform
-                const f32x16 f = f32_block(oa, ob, wm0 + 32 * i, wo0 + 32 * j, kbeg, kend, lane);
-                const bool col = all || ((cols >> l32) & 1u);
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (col || ((rows >> (8 * (r / 4) + 4 * h + r % 4)) & 1u)) out[i][j][r] = f[r];
-            }
+            if (__any(finite != 0.0f)) all |= 1u << (i * FO + j);
+            if (lost && (flags[wm0 / 32 + i] | flags[(BM + wo0) / 32 + j])) redo |= 1u << (i * FO + j);
         }
+    redo = __builtin_amdgcn_readfirstlane(redo | all);
+    // (expected not to be taken: else its scalars are spilled around the k loop)
+    while (__builtin_expect(redo != 0, 0)) {  // uniform
+        const int b = __builtin_ctz(redo), bi = b / FO, bj = b % FO;
+        redo &= redo - 1;
+        const f32x16 f = f32_block(oa, ob, wm0 + 32 * bi, wo0 + 32 * bj, kbeg, kend, lane);
+        const bool every = (all >> b) & 1u;
+        const uint32_t rows = every || !lost ? 0 : flags[wm0 / 32 + bi];
+        const bool col = every || ((flags[(BM + wo0) / 32 + bj] >> l32) & 1u);
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FO; ++j)
+                if (b == i * FO + j) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        if (col || ((rows >> (8 * (r / 4) + 4 * h + r % 4)) & 1u)) out[i][j][r] = f[r];
+                }
+    }
 
     const TileOut<FO> to = tile_out<BM, BN, FO>(p, m0, n0, wm0, wo0, h, l32, slice, batch);
     const float none[1][1][16] = {};
