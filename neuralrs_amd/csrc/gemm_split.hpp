@@ -27,8 +27,10 @@
 //    have met (2^-134 of a row by 2^120 of a column is a normal result), so
 //    the results of every row of A and column of B that dropped any are
 //    replaced, whatever their size;
-//  * a block with a result that is infinite or NaN (an infinite or NaN input,
-//    a value that rounds past bf16's range, or a true overflow) is replaced.
+//  * results that are infinite or NaN (an infinite or NaN input, a value that
+//    rounds past bf16's range, or a true overflow) are replaced.
+// Which instructions a result comes from thus depends on its own row of A and
+// column of B alone: a sample's bits don't change with the others of its batch.
 //
 // A workgroup of WAVES_M x WAVES_N waves owns a BM x BN block of C. Operand
 // tiles of BK k values are loaded to registers one k-tile ahead, split, and
@@ -44,6 +46,7 @@
 // dimension and alignment takes the same path.
 #pragma once
 
+#include <cfloat>
 #include <utility>
 
 #include "gemm_kernel.hpp"
@@ -580,9 +583,9 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
                 }
     }
 
-    // The exceptions: rows and columns with dropped bits, and blocks with a
-    // result that is not finite (bit i * FO + j of `redo` and `all`).
-    uint32_t redo = 0, all = 0;
+    // The exceptions: rows and columns with dropped bits, and results that are
+    // not finite (bit i * FO + j of `redo`: the block has any).
+    uint32_t redo = 0;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -590,18 +593,18 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
             float finite = 0.0f;  // 0 while every result is finite, else NaN
 #pragma unroll
             for (int r = 0; r < 16; ++r) finite = fmaf(out[i][j][r], 0.0f, finite);
-            if (__any(finite != 0.0f)) all |= 1u << (i * FO + j);
-            if (lost && (flags[wm0 / 32 + i] | flags[(BM + wo0) / 32 + j])) redo |= 1u << (i * FO + j);
+            if (__any(finite != 0.0f) ||
+                (lost && (flags[wm0 / 32 + i] | flags[(BM + wo0) / 32 + j])))
+                redo |= 1u << (i * FO + j);
         }
-    redo = __builtin_amdgcn_readfirstlane(redo | all);
+    redo = __builtin_amdgcn_readfirstlane(redo);
     // (expected not to be taken: else its scalars are spilled around the k loop)
     while (__builtin_expect(redo != 0, 0)) {  // uniform
         const int b = __builtin_ctz(redo), bi = b / FO, bj = b % FO;
         redo &= redo - 1;
         const f32x16 f = f32_block(oa, ob, wm0 + 32 * bi, wo0 + 32 * bj, kbeg, kend, lane);
-        const bool every = (all >> b) & 1u;
-        const uint32_t rows = every || !lost ? 0 : flags[wm0 / 32 + bi];
-        const bool col = every || ((flags[(BM + wo0) / 32 + bj] >> l32) & 1u);
+        uint32_t rows = lost ? flags[wm0 / 32 + bi] : 0;
+        if (lost && ((flags[(BM + wo0) / 32 + bj] >> l32) & 1u)) rows = ~0u;
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -609,7 +612,9 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
                 if (b == i * FO + j) {
 #pragma unroll
                     for (int r = 0; r < 16; ++r)
-                        if (col || ((rows >> (8 * (r / 4) + 4 * h + r % 4)) & 1u)) out[i][j][r] = f[r];
+                        if (((rows >> (8 * (r / 4) + 4 * h + r % 4)) & 1u) ||
+                            !(fabsf(out[i][j][r]) <= FLT_MAX))
+                            out[i][j][r] = f[r];
                 }
     }
 

@@ -163,3 +163,20 @@ def test_tiny_times_huge(hip, shape, tiny):
         # (f32 instructions round every product and sum)
         bound = (ks[k] + 72) * 2.0 ** -24 * size[k]
         assert np.all(np.abs(got[k] - want[k]) <= bound), name
+
+
+@pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[1], SHAPES[3], SHAPES[8]], ids=IDS)
+def test_bits_do_not_depend_on_the_other_images(hip, shape):
+    """An image of values that the split cannot hold changes no bit of the
+    other images' outputs and input gradients."""
+    sx, sw, sb, sg = sizes(shape)
+    rng = np.random.default_rng(13 + sum(shape))
+    make = lambda s: rng.standard_normal(s).astype(np.float32)
+    x, w, b, g = make(sx), make(sw), make(sb), make(sg)
+    nan = [np.full(s, np.nan, np.float32) for s in (sx, sw, sb)]
+    y0, dx0, _, _ = run(hip, shape, x, w, b, g, nan, 0.0, 0.0)
+    x[-1, :, 2] *= np.float32(2.0 ** -119)
+    x[-1, 0, 0, 0], g[-1, 1, 0, 0] = np.inf, np.nan
+    g[-1, :, -1] *= np.float32(2.0 ** -125)
+    y1, dx1, _, _ = run(hip, shape, x, w, b, g, nan, 0.0, 0.0)
+    assert np.array_equal(y0[:-1], y1[:-1]) and np.array_equal(dx0[:-1], dx1[:-1])

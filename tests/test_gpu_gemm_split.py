@@ -109,7 +109,7 @@ def test_epilogues_exact(hip, layout, shape):
                                    (4096, 256, 130), (4096, 4096, 48)], ids=IDS)
 def test_infinities_nan_and_overflow(hip, layout, shape):
     """The results that are not finite are those of f32 multiplication and
-    addition, and every other result is untouched by them."""
+    addition, and every other one is exact."""
     rows, cols, inner = shape
     rng = np.random.default_rng(7 * rows + layout)
     small = lambda s: int_matrix(rng, s, 1, 8)  # no zeros: inf * 0 only where put
@@ -199,6 +199,29 @@ def test_tiny_times_huge_in_a_group(hip):
                                (dw.to_host((in_f, out_f)), X.T @ G, np.abs(X.T) @ np.abs(G), batch)):
         # (2^-149: results under f32's smallest normal value)
         assert np.all(np.abs(got - want) <= (k + 8) * 2.0 ** -24 * size + k * 2.0 ** -149)
+
+
+@pytest.mark.parametrize("layout", [NN, NT, TN])
+@pytest.mark.parametrize("shape", [(129, 200, 70), (1000, 1333, 65), (4096, 256, 130), (64, 576, 5000),
+                                   (4096, 4096, 48)], ids=IDS)
+def test_bits_do_not_depend_on_other_rows_and_columns(hip, layout, shape):
+    """Rows of A and columns of B with values that the split cannot hold change
+    no bit of the other rows' and columns' results."""
+    rows, cols, inner = shape
+    rng = np.random.default_rng(rows + layout)
+    make = lambda s: rng.standard_normal(s).astype(np.float32)
+    a, b = operands(layout, rows, cols, inner, make, make)
+    before = gemm(hip, layout, a, b, rows, cols, inner)
+    A, B = (a.T if layout == TN else a), (b.T if layout == NT else b)  # views
+    odd = [3, 40, rows - 2]
+    A[3, 5], A[40] = np.nan, np.inf
+    A[rows - 2] *= np.float32(2.0 ** -119)
+    B[1, cols - 3], B[:, 20] = np.float32(3.4e38), np.float32(2.0 ** -127 * 1.3)
+    after = gemm(hip, layout, a, b, rows, cols, inner)
+    same = np.ones((rows, cols), bool)
+    same[odd] = False
+    same[:, [20, cols - 3]] = False
+    assert np.array_equal(before[same], after[same])
 
 
 def test_bmm_large_items(hip):
