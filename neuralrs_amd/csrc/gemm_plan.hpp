@@ -55,11 +55,28 @@ struct GemmSize {
     int64_t ldb() const { return layout == NRS_NT ? K : N; }
 };
 
-// Whether the 32-bit byte offsets of a staged tile hold (at most 255 rows and a
-// k step), and a row of ones can be built (TN only).
-inline bool split_addressable(const GemmSize& s) {
-    return s.K > 0 && s.lda() < (1 << 21) && s.ldb() < (1 << 21) &&
-           (!s.sum_row || s.layout == NRS_TN);
+// Whether the 32-bit byte offsets of a staged tile hold: within the rows of a
+// tile of an operand contiguous in k, within a k step of another. (64-row tiles
+// reach rows of 8.5 million floats. A wide layer of 512 x 2.5 million over 128
+// takes 2275 us on them and 3324 on the f32 kernel.)
+inline bool split_addressable(const GemmSize& s, int tile) {
+    const SplitShape& t = kSplitShapes[tile];
+    const auto reach = [&](bool contiguous_k, int64_t rows, int64_t ld) {
+        return 4 * (contiguous_k ? (rows - 1) * ld + t.bk : (t.bk - 1) * ld + rows);
+    };
+    return reach(s.layout != NRS_TN, t.bm, s.lda()) <= INT32_MAX &&
+           reach(s.layout == NRS_NT, t.bn, s.ldb()) <= INT32_MAX;
+}
+
+// The group kernel (64x64x32 tiles) takes products of any size it can address
+// (a row of ones is built for TN only).
+inline bool group_takes(const GemmSize& s) {
+    return s.K > 0 && split_addressable(s, S64x64) && (!s.sum_row || s.layout == NRS_TN);
+}
+inline bool any_tile_addresses(const GemmSize& s) {
+    bool any = false;
+    for (int t = 0; t < S_COUNT; ++t) any = any || split_addressable(s, t);
+    return any && s.K > 0 && (!s.sum_row || s.layout == NRS_TN);
 }
 
 // The split GEMM takes dense products of more than 32 rows and columns. The f32
@@ -68,12 +85,9 @@ inline bool split_addressable(const GemmSize& s) {
 // a k step into few tiles (1024 x 1024 over 16: 4.4 us against 4.7; with four
 // tiles a CU the split tiles win again, 4096 x 4096 over 16: 23 against 17).
 inline bool split_takes(const GemmSize& s, int cus) {
-    return s.M > 32 && s.N > 32 && split_addressable(s) &&
+    return s.M > 32 && s.N > 32 && any_tile_addresses(s) &&
            (s.K >= 32 || cdiv(s.M, 64) * cdiv(s.N, 64) * s.batch >= 4 * (int64_t)cus);
 }
-
-// The group kernel (64x64 tiles) takes products of any size it can address.
-inline bool group_takes(const GemmSize& s) { return split_addressable(s); }
 
 // Whether every product of nrs_matmul_shared_lhs_backward fits the group
 // kernel: dx (+)= g . W^T and dW = x^T . g.
@@ -83,14 +97,16 @@ inline bool shared_lhs_fits(int64_t rows, int64_t inner, int64_t cols) {
 }
 
 // The tile of the least estimated time for an unsplit product, and that time
-// in us. `gathered`: a convolution's operand.
+// in us. `gathered`: a convolution's operand; `dense`: a dense product, whose
+// tile must address it.
 inline int cheapest_split_tile(int64_t M, int64_t N, int64_t K, int64_t batch, bool gathered,
-                               int cus, double* time = nullptr) {
+                               int cus, double* time = nullptr, const GemmSize* dense = nullptr) {
     int best = S64x64;
     double least = 1e30;
     for (int t = 0; t < S_COUNT; ++t) {
         const SplitShape& s = kSplitShapes[t];
         const SplitCost& cost = gathered ? s.gathered : s.dense;
+        if (dense && !split_addressable(*dense, t)) continue;
         const int64_t per_cu = cdiv(cdiv(M, s.bm) * cdiv(N, s.bn) * batch, (int64_t)cus);
         const double steps = (double)(cdiv(K, s.bk) * s.bk) / 32.0;
         const double est =
@@ -114,14 +130,14 @@ struct SplitPlan {
 inline SplitPlan plan_split(const GemmSize& s, int cus) {
     const int64_t M = s.M + (s.sum_row ? 1 : 0), N = s.N, K = s.K;
     const int64_t t64 = cdiv(M, 64) * cdiv(N, 64) * s.batch;
-    if (s.split_k && s.batch == 1 && t64 < cus && (2 * t64 <= cus || K >= 2048) && K >= 256) {
+    if (s.split_k && s.batch == 1 && split_addressable(s, S64x64) && t64 < cus && (2 * t64 <= cus || K >= 2048) && K >= 256) {
         const int64_t want = std::min<int64_t>(256, cdiv(3 * (int64_t)cus, t64));
         const int64_t max_by_k = std::max<int64_t>(1, K / ((t64 >= 16 ? 8 : 2) * 32));
         const int64_t slices = std::max<int64_t>(1, std::min(want, max_by_k));
         const int64_t kps = cdiv(cdiv(K, slices), 32) * 32;
         return SplitPlan{S64x64, (int)cdiv(K, kps), kps};
     }
-    const int tile = cheapest_split_tile(M, N, K, s.batch, false, cus);
+    const int tile = cheapest_split_tile(M, N, K, s.batch, false, cus, nullptr, &s);
     const int bk = kSplitShapes[tile].bk;
     return SplitPlan{tile, 1, cdiv(K, bk) * bk};
 }

@@ -37,15 +37,24 @@ def test_planned_tiles_are_addressable(layout):
     assert taken
 
 
+@pytest.mark.parametrize("layout", plan.LAYOUTS)
+def test_wide_matrices_keep_the_split_tiles(layout):
+    """Rows of 2^21 floats and more still run the split GEMM, on the tiles that
+    reach them."""
+    wide = [(512, 2_500_000, 128), (64, 3_000_001, 65), (2_500_000, 512, 128), (100, 90, 4_000_000)]
+    if layout == "NN":  # a k step of 16 rows reaches further
+        wide.append((256, 20_000_000, 32))
+    assert "f32" not in plan.ask(*(("gemm", layout, *s, 1, 0, 1, plan.CUS) for s in wide))
+
+
 def test_shared_lhs_backward_groups_only_what_the_group_kernel_addresses():
-    """Of 64 rows and 8521216 columns, the rows of a gradient tile span 2^31
+    """Of 64 rows and 8.6 million columns, the rows of a gradient tile span 2^31
     bytes: the products have to run one after another."""
-    sizes = [(rows, inner, cols) for rows in (64, 128, 4096) for inner in (64, 256) for cols in EDGES] + \
-            [(64, 64, 8521216)]
+    sizes = [(rows, inner, cols) for rows in (64, 128, 4096) for inner in (64, 256) for cols in EDGES]
     answers = plan.ask(*(("shared", *s) for s in sizes))
     for (rows, inner, cols), answer in zip(sizes, answers):
         if answer == "1":
             assert offsets("NT", rows, inner, cols, (64, 64, 32)) < 1 << 31
             assert offsets("TN", inner, cols, rows, (64, 64, 32)) < 1 << 31
-    assert answers[-1] == "0"
+    assert plan.ask(("shared", 64, 64, 8_600_000)) == ["0"]
     assert plan.ask(("shared", 4096, 256, 256)) == ["1"]
