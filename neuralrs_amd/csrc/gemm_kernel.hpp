@@ -30,6 +30,8 @@
 //    keeps the A rows and B columns those tiles share inside that XCD's L2.
 #pragma once
 
+#include <utility>
+
 #include "buffer_ops.hpp"
 #include "gemm_args.hpp"
 #include "gemm_call.hpp"
@@ -347,6 +349,16 @@ __device__ __forceinline__ TileOut<FN> tile_out(const GemmArgs& p, int64_t m0, i
     return t;
 }
 
+// f(0), .., f(N - 1) with compile-time arguments.
+template <class F, int... I>
+__device__ __forceinline__ void static_for_(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_(f, std::make_integer_sequence<int, N>{});
+}
+
 // The epilogue: bias, ReLU, mask, beta * old and the row of sums. `col0` is
 // the lane's column of fragment j = 0; with EARLY, the old values are passed
 // in (else they are loaded here).
@@ -372,11 +384,22 @@ __device__ __forceinline__ void tile_store(const GemmArgs& p, const TileOut<FN>&
         const bool bias_row = !p.partial && (p.epi & NRS_EPI_BIAS_ROW);
         const bool relu = !p.partial && (p.epi & NRS_EPI_RELU);
         const float* mask = p.partial ? nullptr : p.mask;  // row-major C only
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
+        static_for<FN>([&](auto jc) {  // (a loop this long is not unrolled by its pragma)
+            constexpr int j = decltype(jc)::value;
             const float bc = (bias_col && t.colok[j]) ? p.bias[col0 + 32 * j] : 0.0f;
-#pragma unroll
-            for (int i = 0; i < FM; ++i) {
+            static_for<FM>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                // (opaque, so that nothing is kept from fragment to fragment:
+                // the compiler otherwise holds the addresses and bounds of all
+                // 64 rows of a 128x64 wave tile for its second column of
+                // fragments in scratch memory, more of it than the L2s hold.
+                // 256x256 tiles, us: 200000 x 400 over 32 467, now 130;
+                // 4000 x 4000 over 1000 198, now 158)
+                int64_t st = stride, r0 = row0 + 32 * i;
+                asm volatile("" : "+s"(st), "+v"(r0));
+                const int64_t at0 = t.cbase[j] + r0 * st;  // of element r = 0
+                const int left = (int)min(p.M - r0, (int64_t)32);
+                auto down = [](int r) { return 8 * (r >> 2) + (r & 3); };  // its row, less r0
                 // The fragment's 16 old values and row biases are loaded
                 // before any store, unconditionally from a clamped (always
                 // valid) address: a load inside the store's bounds branch
@@ -387,14 +410,13 @@ __device__ __forceinline__ void tile_store(const GemmArgs& p, const TileOut<FN>&
                 if (beta != 0.0f || bias_row || mask) {  // uniform
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        const int64_t row = row0 + 32 * i + 8 * (r >> 2) + (r & 3);
-                        const bool ok = t.colok[j] & (row < p.M);
+                        const bool ok = t.colok[j] & (down(r) < left);
                         if constexpr (EARLY)
                             old[r] = beta != 0.0f ? early[i][j][r] : 0.0f;
                         else
-                            old[r] = beta != 0.0f ? out[ok ? t.cbase[j] + row * stride : 0] : 0.0f;
-                        br[r] = bias_row ? p.bias[ok ? row : 0] : 0.0f;
-                        live[r] = mask ? mask[ok ? t.cbase[j] + row * stride : 0] > 0.0f : true;
+                            old[r] = beta != 0.0f ? out[ok ? at0 + down(r) * st : 0] : 0.0f;
+                        br[r] = bias_row ? p.bias[ok ? r0 + down(r) : 0] : 0.0f;
+                        live[r] = mask ? mask[ok ? at0 + down(r) * st : 0] > 0.0f : true;
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -416,17 +438,14 @@ __device__ __forceinline__ void tile_store(const GemmArgs& p, const TileOut<FN>&
                     asm volatile("" : "+v"(old[r]));
                 }
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int64_t row = row0 + 32 * i + 8 * (r >> 2) + (r & 3);
-                    if (t.colok[j] && row < p.M) out[t.cbase[j] + row * stride] = old[r];
-                }
+                for (int r = 0; r < 16; ++r)
+                    if (t.colok[j] && down(r) < left) out[at0 + down(r) * st] = old[r];
                 if (p.sum_row) {  // uniform; the row of sums, raw
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        const int64_t row = row0 + 32 * i + 8 * (r >> 2) + (r & 3);
-                        if (t.colok[j] && row == p.M) {
+                        if (t.colok[j] && down(r) == left) {  // (left = 32: no row of sums here)
                             if (p.partial) {
-                                out[t.cbase[j] + row * stride] = acc[i][j][r];
+                                out[at0 + down(r) * st] = acc[i][j][r];
                             } else {
                                 float* sr = p.sum_row + t.cbase[j];
                                 float v = acc[i][j][r];
@@ -436,8 +455,8 @@ __device__ __forceinline__ void tile_store(const GemmArgs& p, const TileOut<FN>&
                         }
                     }
                 }
-            }
-        }
+            });
+        });
     }
 }
 

@@ -47,7 +47,6 @@
 #pragma once
 
 #include <cfloat>
-#include <utility>
 
 #include "gemm_kernel.hpp"
 
@@ -66,16 +65,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // two a matrix instruction halve its rate). The empty asm pins each step's
 // place. Bits of x2 that its bf16 form drops go to `sticky` (low 16 bits).
 constexpr int kSplitSteps = 12;
-
-// f(0), .., f(N - 1) with compile-time arguments.
-template <class F, int... I>
-__device__ __forceinline__ void static_for_(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_(f, std::make_integer_sequence<int, N>{});
-}
 
 struct SplitState {
     float a[4], b[4];       // remainders of the even and the odd floats
