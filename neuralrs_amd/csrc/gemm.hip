@@ -385,6 +385,7 @@ namespace {
 GemmSize size_of(const GemmCall& c) {
     GemmSize s{c.layout, c.M, c.N, c.K, c.batch, c.sum_row != nullptr};
     s.split_k = c.allow_split && c.nchw_P == 0;
+    s.wide = vec4_loads(c);
     return s;
 }
 

@@ -46,11 +46,12 @@ constexpr SplitShape kSplitShapes[S_COUNT] = {
 };
 
 // A dense product: C[M][N] over K, `batch` of them, with or without a row of
-// sums; `split_k` if it may be split over K.
+// sums; `split_k` if it may be split over K, `wide` if the f32 kernels would
+// load it in 128 bits (aligned rows of whole float4s).
 struct GemmSize {
     int layout;
     int64_t M, N, K, batch;
-    bool sum_row = false, split_k = true;
+    bool sum_row = false, split_k = true, wide = false;
     int64_t lda() const { return layout == NRS_TN ? M : K; }
     int64_t ldb() const { return layout == NRS_NT ? K : N; }
 };
@@ -77,16 +78,6 @@ inline bool any_tile_addresses(const GemmSize& s) {
     bool any = false;
     for (int t = 0; t < S_COUNT; ++t) any = any || split_addressable(s, t);
     return any && s.K > 0 && (!s.sum_row || s.layout == NRS_TN);
-}
-
-// The split GEMM takes dense products of more than 32 rows and columns. The f32
-// tiles keep gathered operands, outputs of at most 32 rows or columns
-// (padding would leave the matrix cores nothing to gain) and reductions under
-// a k step into few tiles (1024 x 1024 over 16: 4.4 us against 4.7; with four
-// tiles a CU the split tiles win again, 4096 x 4096 over 16: 23 against 17).
-inline bool split_takes(const GemmSize& s, int cus) {
-    return s.M > 32 && s.N > 32 && any_tile_addresses(s) &&
-           (s.K >= 32 || cdiv(s.M, 64) * cdiv(s.N, 64) * s.batch >= 4 * (int64_t)cus);
 }
 
 // Whether every product of nrs_matmul_shared_lhs_backward fits the group
@@ -118,6 +109,32 @@ inline int cheapest_split_tile(int64_t M, int64_t N, int64_t K, int64_t batch, b
     }
     if (time) *time = least;
     return best;
+}
+
+// Whether a product of a short reduction is ahead on the f32 kernel's 64x64 tile:
+// over at most one of its k steps with 128-bit loads, and up to two where the
+// split's second step is a partial one of an operand contiguous in k, which it
+// loads value by value. Both ways over 38000 products, split against f32 (us):
+//   100 x 50000 over 32 NN 15.9 / 12.5   20860 x 128 over 52 NT 11.0 / 8.5
+//   23 x 638x404 over 24 NT 15.0 / 11.9  over 64 64x64 tiles 0.99x
+//   without 128-bit loads over 32 .. 64 0.70x to 0.97x
+//   256x256 tiles over 32 1.08x, of whole tiles 0.98x, over 16 0.92x
+inline bool f32_ahead(const GemmSize& s, int cus) {
+    if (!s.wide || s.K >= 64) return false;
+    const bool big = cheapest_split_tile(s.M, s.N, s.K, s.batch, false, cus, nullptr, &s) == S256x256;
+    if (big) return s.K > 16 && s.K <= 32 && (s.M % 256 || s.N % 256);
+    return s.K <= 32 || s.layout != NRS_TN;
+}
+
+// The split GEMM takes dense products of more than 32 rows and columns. The f32
+// tiles keep gathered operands, outputs of at most 32 rows or columns
+// (padding would leave the matrix cores nothing to gain), short reductions where
+// they are ahead and those under a k step into few tiles (1024 x 1024 over 16: 4.4
+// us against 4.7; with four tiles a CU the split tiles win again without 128-bit
+// loads).
+inline bool split_takes(const GemmSize& s, int cus) {
+    return s.M > 32 && s.N > 32 && any_tile_addresses(s) && !f32_ahead(s, cus) &&
+           (s.K >= 32 || cdiv(s.M, 64) * cdiv(s.N, 64) * s.batch >= 4 * (int64_t)cus);
 }
 
 struct SplitPlan {

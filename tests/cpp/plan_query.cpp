@@ -1,6 +1,7 @@
 // Answers what the planner of the split GEMM (gemm_plan.hpp) decides, one line
 // of output per line of input. The layouts are NN, NT, TN; sizes are integers.
 //   gemm LAYOUT M N K BATCH ROW_OF_SUMS SPLIT_K CUS  ->  "BMxBNxBK SLICES K_PER_SLICE" or "f32"
+//     (of operands 16-byte aligned)
 //   group LAYOUT M N K ROW_OF_SUMS                   ->  1 if the group kernel takes it
 //   shared ROWS INNER COLS                           ->  1 if the shared-lhs backward runs as a group
 #include <iostream>
@@ -20,7 +21,8 @@ int main() {
             int64_t m, n, k, batch;
             int sums, split, cus;
             in >> layout >> m >> n >> k >> batch >> sums >> split >> cus;
-            const nrs::GemmSize s{layout_of(layout), m, n, k, batch, sums != 0, split != 0};
+            nrs::GemmSize s{layout_of(layout), m, n, k, batch, sums != 0, split != 0};
+            s.wide = s.lda() % 4 == 0 && s.ldb() % 4 == 0 && (batch == 1 || (m * k % 4 == 0 && n * k % 4 == 0));
             if (!nrs::split_takes(s, cus)) {
                 std::cout << "f32\n";
             } else {

@@ -47,6 +47,16 @@ def test_wide_matrices_keep_the_split_tiles(layout):
     assert "f32" not in plan.ask(*(("gemm", layout, *s, 1, 0, 1, plan.CUS) for s in wide))
 
 
+def test_short_reductions_of_aligned_rows_run_the_f32_kernel():
+    """One k step of the f32 kernel, or two of which the split's second would be
+    a partial one read value by value."""
+    f32 = [("NN", 100, 50000, 32, 1), ("NT", 20860, 128, 52, 1), ("NT", 638, 404, 24, 23), ("TN", 2048, 640, 32, 1)]
+    split = [("NN", 100, 50000, 64, 1), ("NT", 20860, 128, 64, 1), ("NT", 637, 404, 33, 23), ("TN", 20860, 128, 52, 1),
+             ("NN", 4096, 4096, 32, 1), ("NN", 4000, 4000, 16, 1), ("TN", 2047, 641, 32, 1)]
+    ask = lambda shapes: plan.ask(*(("gemm", *s, 0, 1, plan.CUS) for s in shapes))
+    assert ask(f32) == ["f32"] * len(f32) and "f32" not in ask(split)
+
+
 def test_shared_lhs_backward_groups_only_what_the_group_kernel_addresses():
     """Of 64 rows and 8.6 million columns, the rows of a gradient tile span 2^31
     bytes: the products have to run one after another."""
