@@ -399,36 +399,43 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * KS, 2) void conv_split_wgr
 }
 
 // dw[m][n] = sum over slices of part[slice][m][n] + beta * dw, n < cols, and
-// db[m] from column cols. 64 outputs and kSumWaves runs of slices a workgroup,
-// the runs added in order: with a thread per output, a small layer's few
-// thousand outputs over 256 slices were one long chain of loads (M 32, 145
-// columns: 12.4 us, now 5).
-constexpr int kSumWaves = 16;
+// db[m] from column cols. A workgroup is groups of `waves` waves, each group 64
+// outputs and a run of slices a wave, the runs added in order: with a thread per
+// output, a small layer's few thousand outputs over 256 slices were one long
+// chain of loads (M 32, 145 columns: 12.4 us, now 5). No more waves than slices:
+// of 16, the 5x5 weight gradient of 256 -> 256 channels over a 7x7 image, 1.6
+// million outputs of one slice, kept 15 idle and took 62 us, with one 22.
+constexpr int kSumWaves = 16, kSumThreads = 256;
 __global__ __launch_bounds__(64 * kSumWaves) void conv_split_sum_kernel(
-    float* dw, float* db, const float* part, int slices, int M, int cols, float beta, FastDiv div_n) {
+    float* dw, float* db, const float* part, int slices, int M, int cols, float beta, FastDiv div_n,
+    int waves) {
     __shared__ float red[kSumWaves][64];
-    const int total = M * (cols + 1), tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int e = blockIdx.x * 64 + tx;
-    const int per = (slices + kSumWaves - 1) / kSumWaves;
+    const int total = M * (cols + 1), tx = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6, ty = wave % waves, group = wave / waves;
+    const int e = (blockIdx.x * (blockDim.x / (64 * waves)) + group) * 64 + tx;
+    const int per = (slices + waves - 1) / waves;
     const int s0 = ty * per, s1 = min(slices, s0 + per);
     const float* src = part + min(e, total - 1);
     float v = 0.0f;
-    for (int s = s0; s < s1; s += 16) {
-        float x[16];
+    if (per <= 2) {  // uniform; short runs without the loads past their end
+        for (int s = s0; s < s1; ++s) v += src[(int64_t)s * total];
+    } else {
+        for (int s = s0; s < s1; s += 16) {
+            float x[16];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = src[(int64_t)min(s + j, s1 - 1) * total];
-        if (s + 8 < s1) {
+            for (int j = 0; j < 8; ++j) x[j] = src[(int64_t)min(s + j, s1 - 1) * total];
+            if (s + 8 < s1) {
 #pragma unroll
-            for (int j = 8; j < 16; ++j) x[j] = src[(int64_t)min(s + j, s1 - 1) * total];
+                for (int j = 8; j < 16; ++j) x[j] = src[(int64_t)min(s + j, s1 - 1) * total];
+            }
+#pragma unroll
+            for (int j = 0; j < 16; ++j) v += s + j < s1 ? x[j] : 0.0f;
         }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) v += s + j < s1 ? x[j] : 0.0f;
     }
-    red[ty][tx] = v;
+    red[wave][tx] = v;
     __syncthreads();
     if (ty || e >= total) return;
-#pragma unroll
-    for (int y = 1; y < kSumWaves; ++y) v += red[y][tx];
+    for (int y = 1; y < waves; ++y) v += red[wave + y][tx];
     uint32_t m, n;
     fast_divmod((uint32_t)e, div_n, m, n);
     float* dst = (int)n < cols ? dw + (int64_t)m * cols + n : (db ? db + m : nullptr);
@@ -577,9 +584,12 @@ int split_wgrad(const SlabWgrad& s) {
     hipLaunchKernelGGL(t.kernel, grid, dim3(t.threads), 0, stream(), a);
     NRS_LAUNCH_CHECK("conv2d weight gradient (split)");
     const int64_t total = s.M * g.N;
-    hipLaunchKernelGGL(conv_split_sum_kernel, dim3((unsigned)cdiv(total, 64)), dim3(64 * kSumWaves), 0,
-                       stream(), s.dw, s.db, g.partial, (int)slices, s.M, (int)cols, s.beta,
-                       make_fastdiv((uint32_t)g.N));
+    int waves = 1;
+    while (waves < kSumWaves && waves < slices) waves *= 2;
+    const int threads = std::max(kSumThreads, 64 * waves);
+    hipLaunchKernelGGL(conv_split_sum_kernel, dim3((unsigned)cdiv(total, threads / waves)), dim3(threads),
+                       0, stream(), s.dw, s.db, g.partial, (int)slices, s.M, (int)cols, s.beta,
+                       make_fastdiv((uint32_t)g.N), waves);
     NRS_LAUNCH_CHECK("conv2d weight gradient (split, sum)");
     return NRS_OK;
 }
