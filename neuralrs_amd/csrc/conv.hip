@@ -1324,6 +1324,36 @@ bool pipe_backward_better(const SlabWgrad& w, bool dinput) {
     return w.N >= 64 && (w.N <= 128 || w.H * w.W >= 100 || w.C <= 32);
 }
 
+// Whether the direct weight gradient of few columns (small_wgrad, a workgroup an
+// image and 4, 2 or 1 channels) is ahead of the split tiles, where 64 channels
+// and 64 columns cost the same however few there are. Both are estimated in us,
+// fitted to 1777 layers of 1 .. 32 columns, 4 .. 128 channels, images 7x7 ..
+// 64x64 and batches of 1 .. 256: the choice is 0.8% from the better one in the
+// mean, and the split tiles alone 4.7%, up to three times: 4->8 1x1 N 208 37^2
+// 14.5 / 44, 1->16 3x3 N 218 63^2 46 / 108, 1->32 N 161 63^2 1x1 53 / 85, but
+// 3->32 3x3 N 32 64^2 121 / 21.
+bool small_wgrad_better(const SlabWgrad& w) {
+    const int64_t taps = (int64_t)w.C * w.kh * w.kw, P = (int64_t)w.OH * w.OW;
+    if (w.N * w.M * (taps + 1) > INT32_MAX) return false;  // (small_wgrad's partials)
+    const int cls = taps <= 9 ? 0 : taps <= 16 ? 1 : 2, channels = 4 >> cls;
+    const double base[3] = {7.2, 8.9, 10.8}, round[3] = {1.28, 2.6, 5.07}, image[3] = {1.9, 6.1, 7.6};
+    const double groups = (double)(w.N * ((w.M + channels - 1) / channels)) / 256, kpx = (double)P / 1000;
+    const double small = base[cls] + round[cls] * groups * (1 + kpx) + image[cls] * kpx;
+    const int64_t quads = w.N * w.OH * ((w.OW + 3) / 4);
+    const double step = w.OW % 4 ? 1.06 : w.stride == 1 && w.pad <= 1 && w.W >= 4 ? 0.7 : 0.88;
+    return small < 9.2 + step * (double)((w.M + 63) / 64) * (double)quads / (8 * 256);
+}
+
+// Whether the im2col lowering (three launches) of a weight gradient past the
+// slab kernel's 18 taps is ahead of the split tiles: a large output over a few
+// hundred pixels, where tiles, partial sums and their launch are all there is.
+// 5x5, im2col against split (us): 256->256 N 2 5^2 14.5 / 23, 128->256 N 1 21^2
+// stride 2 14.6 / 23, 128->128 N 1 24^2 22 / 19, 256->256 N 3 19^2 60 / 36.
+bool im2col_wgrad_better(const SlabWgrad& w) {
+    const int64_t taps = (int64_t)w.kh * w.kw;
+    return taps > 18 && w.N * w.OH * w.OW <= 400 && w.M * (w.C * taps + 1) >= 1 << 17;
+}
+
 // Whether the slab weight gradient on its own is: many small images, above all
 // of rows that are no whole quads, whose pixels the split tiles gather one by
 // one. Slab against split (us): N 256 16->32 7^2 15 / 18; 10^2 N 128 32->32
@@ -1347,12 +1377,16 @@ bool slab_wgrad_better(const SlabWgrad& w) {
 // N 256 64->20 48 / 40. Larger images come in bands: 16^2 N 64 32->64 33 / 41,
 // 8->64 30 / 29, N 128 43 / 33. Up to 32 input channels the split tiles do not
 // take the input gradient, and on its own over many gradient channels it is one
-// long chain a workgroup: 32->96 N 24 15^2 37 / 66, N 8 40^2 47 / 57.
+// long chain a workgroup: 32->96 N 24 15^2 37 / 66, N 8 40^2 47 / 57. With up to
+// 16 it stays ahead until the gradient outgrows the pair's launch: 8->256 N 4 45^2
+// 61 / 83, 16->128 N 1 20^2 37 / 50, 16->96 N 2 54^2 41 / 55, but 8->256 N 16 32^2
+// 98 / 80.
 bool slab_pair_better(const SlabWgrad& w) {
     const int64_t pixels = (int64_t)w.H * w.W, size = (int64_t)w.C * w.C * w.M * w.N;
     const int taps = w.kh * w.kw;
     if (taps > 9 || w.stride != 1) return false;
     if (taps > 1 && w.M > 64 && w.C > 16 && w.C <= 32 && w.N * pixels <= 16384) return true;
+    if (taps > 1 && w.M > 64 && w.C <= 16 && w.N * pixels * w.M <= 4 << 20) return true;
     if (w.H > 16 || w.W > 16) return false;
     if (pixels <= (w.OW % 4 ? 225 : 196) && size <= (taps == 1 && pixels <= 100 ? 20 : 15) << 20) return true;
     if (w.C * w.M <= 512) return pixels <= 64 || (w.N > 128 && pixels <= 196);
@@ -1984,15 +2018,18 @@ int nrs_conv2d_backward_ex(float* dinput, float* dweight, float* dbias, const fl
         f.OW = (int)d.out_w;
         f.beta = beta_params;
         if ((rc = nrs::few_taps_wgrad(f)) != nrs::kSlabUnsupported) return rc;
-        if (fits_w && (rc = nrs::split_wgrad(w)) != nrs::kSlabUnsupported) return rc;
-        // (a bias gradient alone, or tensors past the split tiles' 2 GiB)
+        if (fits_w && !nrs::small_wgrad_better(w) &&
+            (rc = nrs::split_wgrad(w)) != nrs::kSlabUnsupported)
+            return rc;
+        // (also a bias gradient alone, and tensors past the split tiles' 2 GiB)
         return nrs::small_wgrad(dweight, dbias, grad, input, d, beta_params);
     }
     if (slab_w) {
         if (nrs::pipe_backward_better(w, false) &&
             (rc = nrs::pipe_backward(nullptr, w)) != nrs::kSlabUnsupported)
             return rc;
-        if (!nrs::slab_wgrad_better(w) && (rc = nrs::split_wgrad(w)) != nrs::kSlabUnsupported)
+        if (!nrs::slab_wgrad_better(w) && !nrs::im2col_wgrad_better(w) &&
+            (rc = nrs::split_wgrad(w)) != nrs::kSlabUnsupported)
             return rc;
         // input slab and gradient rows staged in LDS, reduction on the matrix
         // cores, per-slice partials summed in a fixed order (also tensors past
