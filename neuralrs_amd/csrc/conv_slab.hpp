@@ -1,29 +1,12 @@
-// Slab-resident convolution: host-side interface (kernel in conv_slab.hip).
-//
-// out[n, m, oy, ox] = sum_{c,i,j} x[n, c, oy*s - pad_h + i, ox*s - pad_w + j] * Wt(m, c, i, j)
-//                     (+ bias[m]) + beta * out
-// with Wt(m, c, i, j) = w[m][c][i][j] (forward), or, with `flip`, the
-// flipped, channel-transposed w[c][m][kh-1-i][kw-1-j] (the stride-1 input
-// gradient of a convolution with weights w, read as a forward convolution of
-// the output gradient).
+// Convolution kernels: host-side interfaces (what they compute is in
+// conv_plan.hpp, the slab kernel in conv_slab.hip).
 #pragma once
 
+#include "conv_plan.hpp"
 #include "fastdiv.hpp"
 #include "nrs_internal.hpp"
 
 namespace nrs {
-
-struct SlabConv {
-    const float* x = nullptr;     // NCHW [N][C][H][W]
-    const float* w = nullptr;     // [M][C][kh][kw], or [C][M][kh][kw] with flip
-    const float* bias = nullptr;  // [M] or null
-    float* out = nullptr;         // NCHW [N][M][OH][OW]
-    int64_t N = 0;
-    int C = 0, H = 0, W = 0, M = 0, kh = 0, kw = 0, stride = 1, pad_h = 0, pad_w = 0;
-    int OH = 0, OW = 0;
-    bool flip = false;
-    float beta = 0.0f;
-};
 
 // Launches the convolution when its tiles fit the slab kernel's limits and
 // returns NRS_OK; returns kSlabUnsupported (launching nothing) when they do
@@ -50,19 +33,9 @@ int wino_conv(const SlabConv& s);
 // nothing) for other shapes.
 int pipe_conv(const SlabConv& s);
 
-// Weight gradient dw[m][c][i][j] += sum g[n,m,oy,ox] * x[n,c,oy*s-pad+i,ox*s-pad+j]
-// and, when db is given, bias gradient db[m] += sum g[n,m,oy,ox], with
-// per-image partial sums added in a fixed order. dw is required; returns
-// kSlabUnsupported (launching nothing) for shapes outside the kernel's limits.
-struct SlabWgrad {
-    const float* x = nullptr;  // NCHW [N][C][H][W]
-    const float* g = nullptr;  // NCHW [N][M][OH][OW]
-    float* dw = nullptr;       // [M][C][kh][kw]
-    float* db = nullptr;       // [M] or null
-    int64_t N = 0;
-    int C = 0, H = 0, W = 0, M = 0, kh = 0, kw = 0, stride = 1, pad = 0, OH = 0, OW = 0;
-    float beta = 1.0f;  // dw = gradient + beta * dw (likewise db); 0 reads nothing
-};
+// The weight gradient w (dw required), per-image partial sums added in a fixed
+// order; returns kSlabUnsupported (launching nothing) for shapes outside the
+// kernel's limits.
 int slab_wgrad(const SlabWgrad& s);
 
 // The stride-1 input gradient d (a slab convolution with flip) and the

@@ -475,12 +475,8 @@ WgradTile wgrad_tile(int64_t M, int64_t N, int form) {
 }  // namespace
 
 int split_conv(const SlabConv& s) {
+    if (!split_conv_takes(s)) return kSlabUnsupported;
     const int64_t taps = (int64_t)s.kh * s.kw, P = (int64_t)s.OH * s.OW, pixels = s.N * P;
-    const int64_t in_bytes = s.N * s.C * s.H * s.W * 4 + ((int64_t)s.pad_h * s.W + s.pad_w) * 4;
-    // (the taps of the padded last k step must stay within the mask's bits)
-    if (s.C % 4 || cdiv(taps * s.C, 64) * 64 / s.C > 31 || s.M <= 32 || pixels < 64 || pixels > INT32_MAX ||
-        in_bytes > 0x7fffffffll || (int64_t)s.M * s.C * taps > (1 << 28) || s.pad_h < 0 || s.pad_w < 0)
-        return kSlabUnsupported;
     ConvSplitArgs a{};
     GemmArgs& g = a.g;
     g.B = s.x;
@@ -509,8 +505,7 @@ int split_conv(const SlabConv& s) {
     a.div_kw = make_fastdiv((uint32_t)s.kw);
     a.div_p = make_fastdiv((uint32_t)P);
     a.div_ow = make_fastdiv((uint32_t)s.OW);
-    int tile = split_tile_for(s.M, pixels, g.K, 1, true);
-    if (tile == S256x256) tile = S128x128;
+    const int tile = split_conv_tile(s, num_cus());
     const int bm = tile == S128x128 ? 128 : 64, bn = tile == S64x64K || tile == S64x64 ? 64 : 128;
     g.tiles_m = (int)cdiv(s.M, bm);
     g.tiles_n = (int)cdiv(pixels, bn);

@@ -400,14 +400,6 @@ bool groupable(const GemmCall& c) {
            c.partial_buf == nullptr && group_takes(size_of(c));
 }
 
-}  // namespace
-
-int split_tile_for(int64_t M, int64_t N, int64_t K, int64_t batch, bool gathered, double* time) {
-    return cheapest_split_tile(M, N, K, batch, gathered, num_cus(), time);
-}
-
-namespace {
-
 Plan split_plan(const GemmCall& c) {
     const SplitPlan p = plan_split(size_of(c), num_cus());
     return Plan{p.tile, p.slices, p.k_per_slice, 0};

@@ -91,12 +91,6 @@ struct OperandRange {
 // or operands (A, B, bias, extra[j] of call j when extra is non-null).
 bool outputs_independent(const GemmCall* calls, int count, const OperandRange* extra);
 
-// The split GEMM's tile (SplitTile, gemm_plan.hpp) of the least estimated time
-// for `batch` unsplit products of M x N over K, and that time in us; `gathered`
-// products have a convolution's operand.
-int split_tile_for(int64_t M, int64_t N, int64_t K, int64_t batch, bool gathered,
-                   double* time = nullptr);
-
 // Batched products of small dense items (M, N, K <= 128, 16-byte aligned
 // items, K or the transposed operand's rows in whole float4s), without
 // epilogue; returns kBmmUnsupported (launching nothing) for any other call.

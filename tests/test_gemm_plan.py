@@ -25,6 +25,19 @@ EDGES = [(1 << e) + d for e in range(19, 28) for d in (-3, 0, 5)]
 
 
 @pytest.mark.parametrize("layout", plan.LAYOUTS)
+def test_the_products_of_the_gpu_tests_reach_their_tiles(layout):
+    answers = plan.ask(*(("gemm", layout, *shape, 1, 0, 1, plan.CUS) for shape, _ in plan.TILES))
+    for (shape, tile), answer in zip(plan.TILES, answers):
+        assert answer.split()[:2] == [tile, "1"], (shape, answer)
+
+
+def test_the_layers_of_the_gpu_tests_reach_their_tiles():
+    answers = plan.ask(*(("conv", *shape, plan.CUS) for shape, _, _ in plan.CONV_TILES))
+    for (shape, forward, backward), answer in zip(plan.CONV_TILES, answers):
+        assert answer.split() == [forward, backward], (shape, answer)
+
+
+@pytest.mark.parametrize("layout", plan.LAYOUTS)
 def test_planned_tiles_are_addressable(layout):
     sizes = [(m, n, k) for big in EDGES for m, n, k in
              [(64, 64, big), (4096, 4096, big), (big, 64, 64), (64, big, 64), (big, 512, 512), (512, big, 512)]]
