@@ -32,6 +32,9 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_FP32_MFMA_TFLOPS = 157.3   # MI355X dense FP32 matrix peak
+PEAK_BF16_MFMA_TFLOPS = 2500.0  # MI355X dense bf16 matrix peak
+# f32 products on the bf16 matrix cores: six products of bf16 pieces each
+PEAK_F32_PRODUCT_TFLOPS = PEAK_BF16_MFMA_TFLOPS / 6
 PEAK_HBM_GBS = 8000.0           # MI355X HBM3E
 
 
@@ -82,8 +85,9 @@ def leg_ms(hip, fn, reps, warmup, rounds=3):
 
 
 def roofline_us(flops, nbytes):
-    """max(FLOP / FP32 MFMA peak, bytes / HBM bandwidth) in microseconds."""
-    return max(flops / (PEAK_FP32_MFMA_TFLOPS * 1e12), nbytes / (PEAK_HBM_GBS * 1e9)) * 1e6
+    """max(f32 FLOP / the matrix cores' rate for split f32 products, bytes / HBM
+    bandwidth) in microseconds."""
+    return max(flops / (PEAK_F32_PRODUCT_TFLOPS * 1e12), nbytes / (PEAK_HBM_GBS * 1e9)) * 1e6
 
 
 def gemm_roof(m, n, k, batch=1):
@@ -439,11 +443,10 @@ def bench_attention_cfg4(hip, steps, warmup, closures_only=False):
         # sums read grad and x_norm: 9 passes of 4 MB
         ln_roof = roofline_us(0.0, 9 * 4.0 * Rh * Hh * Dh)
     bmm_roof = 6 * roofline_us(*gemm_roof(T, T, Dh, BH))  # every product moves 25.2 MB
-    # the fused core's bound: the six products' FLOP at MFMA peak (forward
-    # 2, backward 4; its HBM traffic, Q/K/V/dO in and O/dQ/dK/dV out, 32 MB,
-    # takes less at 8 TB/s); the backward's recomputation of the scores is
-    # extra work, not counted
-    fused_roof = 6 * 2.0 * BH * T * T * Dh / (PEAK_FP32_MFMA_TFLOPS * 1e12) * 1e6
+    # the fused core's bound: the six products' FLOP (forward 2, backward 4) or
+    # its HBM traffic, Q/K/V/dO in and O/dQ/dK/dV out, 32 MB; the backward's
+    # recomputation of the scores is extra work, not counted
+    fused_roof = roofline_us(6 * 2.0 * BH * T * T * Dh, 8 * 4.0 * BH * T * Dh)
 
     # the block's Linear GEMMs: X[4096,256] through 4 projections and the FFN,
     # launched as the operator surface launches them: the Q, K, V projections
@@ -520,7 +523,7 @@ def bench_sweep_cfg5(hip, reps):
         fl, by = gemm_roof(m, n, k)
         roof = roofline_us(fl, by)
         out[name] = {"us": round(ms * 1e3, 2), "tflops": round(fl / (ms * 1e-3) / 1e12, 2),
-                     "bound": "hbm" if by / (PEAK_HBM_GBS * 1e9) > fl / (PEAK_FP32_MFMA_TFLOPS * 1e12) else "mfma",
+                     "bound": "hbm" if by / (PEAK_HBM_GBS * 1e9) > fl / (PEAK_F32_PRODUCT_TFLOPS * 1e12) else "mfma",
                      "roofline_frac": round(roof / (ms * 1e3), 4), "max_rel_err_vs_f64": err}
         del dA, dB, dC
     return out
@@ -719,6 +722,15 @@ def counters_pass(hip):
         else:
             fn = (lambda a=a, b=b, c=c, m=m, n=n, k=k: hip.gemm_nt_splitk(c, a, b, m, n, k))
         legs.append((name, fn))
+    # a layer of the split convolutions: 64 -> 128 channels, 3x3, 32 images of 32x32
+    dims = (32, 64, 32, 32, 128, 3, 3, 1, 1)
+    x, w, bias, g = (hip.DeviceBuffer.from_host(rng.uniform(-1, 1, s).astype(np.float32))
+                     for s in (32 * 64 * 1024, 128 * 64 * 9, 128, 32 * 128 * 1024))
+    y, dx, dw, db = (hip.DeviceBuffer(s) for s in (32 * 128 * 1024, 32 * 64 * 1024, 128 * 64 * 9, 128))
+    keep += [x, w, bias, g, y, dx, dw, db]
+    legs.append(("conv_64_128_32x32_fwd", lambda: hip.call("nrs_conv2d_forward", y, x, w, bias, *dims)))
+    legs.append(("conv_64_128_32x32_bwd", lambda: hip.call("nrs_conv2d_backward_ex", dx, dw, db, g, x, w,
+                                                           *dims, 0.0, 0.0)))
     legs += list(bench_conv_cfg3(hip, 0, 0, closures_only=True).items())
     legs += list(bench_attention_cfg4(hip, 0, 0, closures_only=True).items())
     legs += list(bench_mlp_cfg2(hip, 0, 0, closures_only=True).items())
@@ -801,9 +813,11 @@ def main():
         "pct_fp32_mfma_peak": round(100.0 * value / PEAK_FP32_MFMA_TFLOPS, 2),
         "max_rel_err_vs_f64": g["rel_err"],
         "roofline": {"bound": "mfma", "achieved": round(achieved, 3),
-                     "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(achieved / PEAK_FP32_MFMA_TFLOPS, 4), "traffic": traffic,
-                     "kernel": "gemm_kernel 256x256x32 tile, 2x4 waves, NN",
+                     "peak": round(PEAK_F32_PRODUCT_TFLOPS, 1), "unit": "TFLOP/s",
+                     "peak_is": "dense bf16 matrix peak / 6 (f32 products as six products of "
+                                "bf16 pieces, f32 accumulation)",
+                     "frac": round(achieved / PEAK_F32_PRODUCT_TFLOPS, 4), "traffic": traffic,
+                     "kernel": "gemm_split_kernel 256x256x16 tile, 2x4 waves, NN",
                      "kernel_ms": round(g["kernel_ms"], 4)},
     }
     if not args.no_conv:
@@ -857,7 +871,7 @@ def main():
                 "timing": "C++ issue (neuralrs_amd/bench_host mlp), HIP events on the stream"})
         hb = host_step("block", 200, 20)
         if hb:
-            gemm_roof = hb["gemm_flop_per_step"] / (PEAK_FP32_MFMA_TFLOPS * 1e12) * 1e6
+            gemm_roof = hb["gemm_flop_per_step"] / (PEAK_F32_PRODUCT_TFLOPS * 1e12) * 1e6
             out["transformer_block_cfg4"] = {
                 "step_us": round(hb["step_gpu_us"], 2), "fwd_us": round(hb["fwd_gpu_us"], 2),
                 "gemm_flop_per_step": hb["gemm_flop_per_step"],

@@ -45,14 +45,14 @@ SHAPES = [  # (rows, cols, inner)
     (512, 512, 512), (32, 1024, 512), (1, 513, 257), (1000, 3, 2),
     (130, 17, 33), (257, 32, 96),  # at most 32 columns: 128x32 tiles, ragged rows
     (2048, 2048, 40), (4096, 1024, 72), (2000, 2048, 36),  # large outputs (the last ragged M)
-    (2000, 2100, 1100),  # 128x128 tiles (one per CU), ragged edges
+    (2000, 2100, 1100),  # several tiles a CU, ragged edges, 128-bit loads
     (30, 8200, 1024),    # at most 32 rows: 32x256 tiles over K slices, ragged M and N
     # cfg4 Linear GEMMs (TransformerBlock, B32 S128 d256 dff1024): Q/K/V/O
     # projections and the two FFN layers forward (NN) and their input
     # gradients (NT); the weight gradients over K = 4096 rows (TN, split-K)
     (4096, 256, 256), (4096, 1024, 256), (4096, 256, 1024),
     (256, 256, 4096), (256, 1024, 4096), (1024, 256, 4096),
-    # k-split wave sets (64x64 tiles, 8 waves) with ragged edges
+    # 64x64 tiles with ragged edges
     (1000, 260, 200), (4000, 300, 96),
 ]
 
@@ -90,9 +90,9 @@ def test_gemm_f64_tolerance(hip, orc, layout, shape):
 @pytest.mark.parametrize("shape", [(4096, 4096, 32), (4096, 4096, 288), (4096, 8192, 96),
                                    (4096, 4096, 100)], ids=lambda s: "x".join(map(str, s)))
 def test_gemm_large_whole_tiles_exact(hip, layout, shape):
-    """Plain products over whole 256x256 tiles that fill the GPU (the
-    256x256 tile, with a K tail at K = 100), all three layouts: exact on
-    small integers, every element."""
+    """Plain products over whole 256x256 tiles that fill the GPU (with a K
+    tail at K = 100), all three layouts: exact on small integers, every
+    element."""
     rows, cols, inner = shape
     rng = np.random.default_rng(rows + cols + inner + layout)
     a, b = operands(layout, rows, cols, inner, lambda s: int_matrix(rng, s, -4, 4))
@@ -144,7 +144,7 @@ def test_gemm_skinny_cfg5(hip, orc):
 
 @pytest.mark.parametrize("shape", [(70, 50, 33), (2000, 2100, 1100), (300, 20, 40), (30, 600, 1024),
                                    (4096, 4096, 64), (1000, 260, 200)],
-                         ids=["64x64", "128x128", "128x32", "32x256-splitk", "256x256", "64x64-ksplit"])
+                         ids=["short", "large-ragged", "128x32", "32x256-splitk", "large", "64x64-ragged"])
 def test_gemm_beta_bias_relu_epilogues(hip, shape):
     """The general epilogue (beta, column bias, row bias + ReLU) on each tile."""
     rng = np.random.default_rng(9)
