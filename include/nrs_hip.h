@@ -22,6 +22,17 @@
  *     (e.g. "cuda matmul: inner dims mismatch", src/cuda/graph/matmul.rs:398);
  *     the host wrapper turns a non-zero code into that panic/exception.
  *   - Not thread-safe (the reference's host side is Rc<RefCell>, !Send).
+ *   - Products: f32 operands, f32 sums, in an order that depends on the sizes
+ *     and the operands' alignment alone, so the same call gives the same bits
+ *     and a row of a result does not depend on the other rows' values. Larger products (of more than 32
+ *     rows and columns, and convolutions past the small kernels) represent
+ *     each float exactly in three bf16 pieces and add six of the nine products
+ *     of pieces; the other three are at most 2^-24 of a product, so a result of
+ *     one or two terms may be off by up to 2 * 2^-24 of it where an f32
+ *     multiply is by 2^-24, and longer sums are as close to the exact one as
+ *     f32 multiply-adds or closer. Values that pieces cannot hold (infinities,
+ *     NaN, magnitudes under 2^-110 or near the largest float) are multiplied in
+ *     f32: such rows cost up to three times an ordinary call.
  */
 #ifndef NRS_HIP_H
 #define NRS_HIP_H
@@ -103,11 +114,11 @@ int nrs_gemm(int layout, float *C, const float *A, const float *B,
  * and matmul_tn for dB, each followed by accumulate_into) or the projections
  * of one input (src/cuda/nn/multihead.rs:64-66, three matmuls of x). Each
  * descriptor means exactly nrs_gemm with its fields; at most
- * NRS_GEMM_GROUP_MAX of them. When every call is dense, 16-byte aligned with
- * rows of whole float4s and no output overlaps another call's output or
- * operands, their workgroups share one grid (one problem's load latency,
- * barriers and epilogue overlap another's matrix-core work); otherwise the
- * calls run one after another in the order given. Results equal nrs_gemm's to
+ * NRS_GEMM_GROUP_MAX of them. When every call is dense and within the grouped
+ * kernel's 32-bit tile offsets (rows under 8.5 million floats), and no output
+ * overlaps another call's output or operands, their workgroups share one grid
+ * (one problem's load latency, barriers and epilogue overlap another's
+ * matrix-core work); otherwise the calls run one after another in the order given. Results equal nrs_gemm's to
  * the GEMM tolerance (the tiling, hence the summation order, may differ).   */
 #define NRS_GEMM_GROUP_MAX 4
 typedef struct nrs_gemm_desc {
