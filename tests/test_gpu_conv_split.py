@@ -54,6 +54,11 @@ SHAPES = [  # n, c_in, c_out, h, w, kh, kw, stride, pad
     (1, 16, 32, 5, 6, 3, 3, 1, 0),
     (1, 9, 70, 1, 4, 3, 3, 1, 1),        # one output row of one quad
     (3, 256, 160, 7, 7, 3, 3, 1, 1),
+    # layers that the rules leave to the kernels before the split tiles: a weight
+    # gradient of few columns, of many over few pixels, and the backward pair
+    (30, 4, 8, 21, 23, 1, 1, 1, 0),
+    (2, 64, 128, 6, 5, 5, 5, 1, 2),
+    (1, 16, 128, 20, 20, 3, 3, 1, 1),
 ]
 WIDE = [shape for shape, _, _ in plan.CONV_TILES]
 IDS = lambda s: "x".join(map(str, s))
