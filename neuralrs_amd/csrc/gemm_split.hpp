@@ -28,11 +28,11 @@
 // x2 may need bits under bf16's smallest denormal) whose x0 is finite. Both
 // exceptions are seen and computed again on the f32 instructions, 32x32 blocks
 // of C at a time, from global memory (f32_block):
-//  * staging keeps, for every unit, the OR of the bits of its x2s that their
-//    bf16 form drops. How much those bits matter depends on what they would
-//    have met (2^-134 of a row by 2^120 of a column is a normal result), so
-//    the results of every row of A and column of B that dropped any are
-//    replaced, whatever their size;
+//  * staging keeps, for every row a thread stages units of, the OR of the bits
+//    of its x2s that their bf16 form drops. How much those bits matter depends
+//    on what they would have met (2^-134 of a row by 2^120 of a column is a
+//    normal result), so the results of every row of A and column of B that
+//    dropped any are replaced, whatever their size;
 //  * results that are infinite or NaN (an infinite or NaN input, a value that
 //    rounds past bf16's range, or a true overflow) are replaced.
 // Which instructions a result comes from thus depends on its own row of A and
@@ -362,9 +362,18 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
     constexpr bool kMasked = OA::kMasked && OB::kMasked;
     const int nfull = kMasked ? ntiles : (int)((kend - kbeg) / BK);
     constexpr int kUnits = C_::UA + C_::UB;
-    uint32_t sticky[kUnits];
+    // One word for all of a thread's units where they are of one row: with a word
+    // each, the registers that the 64x128 convolution tile had left cost it 6%
+    // (128 -> 128 channels 3x3, N 21 20^2: 48.1 us, shared 44.8).
+    constexpr int kFirstB = !OA::kKC && NT % BM == 0 ? 1 : C_::UA;
+    constexpr int kSticky = kFirstB + (!OB::kKC && NT % BN == 0 ? 1 : C_::UB);
+    auto word = [](int un) constexpr {
+        return un < C_::UA ? (un < kFirstB ? un : kFirstB - 1)
+                           : (un - C_::UA < kSticky - kFirstB ? kFirstB + un - C_::UA : kSticky - 1);
+    };
+    uint32_t sticky[kSticky];
 #pragma unroll
-    for (int un = 0; un < kUnits; ++un) sticky[un] = 0;
+    for (int w = 0; w < kSticky; ++w) sticky[w] = 0;
     auto load_unit = [&](int t, int un, auto part) {
         constexpr bool PART = decltype(part)::value;
         const int64_t k0 = kbeg + (int64_t)t * BK;
@@ -397,7 +406,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
         constexpr bool in_a = un < C_::UA;
         constexpr int i = in_a ? un : un - C_::UA;
         if constexpr (!in_a && OB::kFix && x % kSplitSteps == 0) ob.fix(rb[i], i);
-        st.template step<x % kSplitSteps>(in_a ? ra[i] : rb[i], sticky[un],
+        st.template step<x % kSplitSteps>(in_a ? ra[i] : rb[i], sticky[word(un)],
                                           in_a ? OA::kOnes && ((oa.ones >> i) & 1u)
                                                : OB::kOnes && ((ob.ones >> i) & 1u));
         if constexpr (x % kSplitSteps == kSplitSteps - 1) {
@@ -517,7 +526,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
     }
     uint32_t dropped = 0;
 #pragma unroll
-    for (int un = 0; un < kUnits; ++un) dropped |= sticky[un];
+    for (int w = 0; w < kSticky; ++w) dropped |= sticky[w];
     const bool lost = __syncthreads_or((int)(dropped & 0xffffu));
     // (the barrier above: every wave is done with the staging buffers)
     // A bit for each row and column of the tile with dropped bits, past what
@@ -535,7 +544,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, u32x4* smem, OA& o
             else
                 split_pos<BN, BK, OB::kKC, NT>(un - C_::UA, tid, row, q);
             if (un >= C_::UA) row += BM;
-            if (sticky[un] & 0xffffu) atomicOr(flags + row / 32, 1u << (row % 32));
+            if (sticky[word(un)] & 0xffffu) atomicOr(flags + row / 32, 1u << (row % 32));
         }
         __syncthreads();
     }
