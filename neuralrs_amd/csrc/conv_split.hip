@@ -399,21 +399,25 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * KS, 2) void conv_split_wgr
 }
 
 // dw[m][n] = sum over slices of part[slice][m][n] + beta * dw, n < cols, and
-// db[m] from column cols. A workgroup is groups of `waves` waves, each group 64
+// db[m] from column cols. A workgroup is groups of WAVES waves, each group 64
 // outputs and a run of slices a wave, the runs added in order: with a thread per
 // output, a small layer's few thousand outputs over 256 slices were one long
 // chain of loads (M 32, 145 columns: 12.4 us, now 5). No more waves than slices:
 // of 16, the 5x5 weight gradient of 256 -> 256 channels over a 7x7 image, 1.6
-// million outputs of one slice, kept 15 idle and took 62 us, with one 22.
-constexpr int kSumWaves = 16, kSumThreads = 256;
-__global__ __launch_bounds__(64 * kSumWaves) void conv_split_sum_kernel(
-    float* dw, float* db, const float* part, int slices, int M, int cols, float beta, FastDiv div_n,
-    int waves) {
-    __shared__ float red[kSumWaves][64];
+// million outputs of one slice, kept 15 idle and took 62 us, with one 22. WAVES
+// is the kernel's own, so that a group's runs are read from LDS together: with a
+// loop of unknown length 110,720 outputs of 16 slices took 8.9 us, now 6.6.
+constexpr int kSumWaves = 16;
+constexpr int sum_threads(int waves) { return waves < 4 ? 256 : 64 * waves; }
+template <int WAVES>
+__global__ __launch_bounds__(sum_threads(WAVES)) void conv_split_sum_kernel(
+    float* dw, float* db, const float* part, int slices, int M, int cols, float beta, FastDiv div_n) {
+    constexpr int kGroups = sum_threads(WAVES) / (64 * WAVES);
+    __shared__ float red[kGroups * WAVES][64];
     const int total = M * (cols + 1), tx = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6, ty = wave % waves, group = wave / waves;
-    const int e = (blockIdx.x * (blockDim.x / (64 * waves)) + group) * 64 + tx;
-    const int per = (slices + waves - 1) / waves;
+    const int wave = threadIdx.x >> 6, ty = wave % WAVES, group = wave / WAVES;
+    const int e = (blockIdx.x * kGroups + group) * 64 + tx;
+    const int per = (slices + WAVES - 1) / WAVES;
     const int s0 = ty * per, s1 = min(slices, s0 + per);
     const float* src = part + min(e, total - 1);
     float v = 0.0f;
@@ -435,11 +439,23 @@ __global__ __launch_bounds__(64 * kSumWaves) void conv_split_sum_kernel(
     red[wave][tx] = v;
     __syncthreads();
     if (ty || e >= total) return;
-    for (int y = 1; y < waves; ++y) v += red[wave + y][tx];
+#pragma unroll
+    for (int y = 1; y < WAVES; ++y) v += red[wave + y][tx];
     uint32_t m, n;
     fast_divmod((uint32_t)e, div_n, m, n);
     float* dst = (int)n < cols ? dw + (int64_t)m * cols + n : (db ? db + m : nullptr);
     if (dst) *dst = beta != 0.0f ? v + beta * *dst : v;
+}
+
+using SumKernel = void (*)(float*, float*, const float*, int, int, int, float, FastDiv);
+SumKernel sum_kernel(int waves) {
+    switch (waves) {
+        case 1: return conv_split_sum_kernel<1>;
+        case 2: return conv_split_sum_kernel<2>;
+        case 4: return conv_split_sum_kernel<4>;
+        case 8: return conv_split_sum_kernel<8>;
+        default: return conv_split_sum_kernel<kSumWaves>;
+    }
 }
 
 using WgradKernel = void (*)(ConvSplitArgs);
@@ -581,10 +597,10 @@ int split_wgrad(const SlabWgrad& s) {
     const int64_t total = s.M * g.N;
     int waves = 1;
     while (waves < kSumWaves && waves < slices) waves *= 2;
-    const int threads = std::max(kSumThreads, 64 * waves);
-    hipLaunchKernelGGL(conv_split_sum_kernel, dim3((unsigned)cdiv(total, threads / waves)), dim3(threads),
-                       0, stream(), s.dw, s.db, g.partial, (int)slices, s.M, (int)cols, s.beta,
-                       make_fastdiv((uint32_t)g.N), waves);
+    const int threads = sum_threads(waves);
+    hipLaunchKernelGGL(sum_kernel(waves), dim3((unsigned)cdiv(total, threads / waves)), dim3(threads), 0,
+                       stream(), s.dw, s.db, g.partial, (int)slices, s.M, (int)cols, s.beta,
+                       make_fastdiv((uint32_t)g.N));
     NRS_LAUNCH_CHECK("conv2d weight gradient (split, sum)");
     return NRS_OK;
 }
