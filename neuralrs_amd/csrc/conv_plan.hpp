@@ -161,15 +161,20 @@ inline bool slab_wgrad_better(const SlabWgrad& w) {
 // 8->64 30 / 29, N 128 43 / 33. Up to 32 input channels the split tiles do not
 // take the input gradient, and on its own over many gradient channels it is one
 // long chain a workgroup: 32->96 N 24 15^2 37 / 66, N 8 40^2 47 / 57. With up to
-// 16 it stays ahead until the gradient outgrows the pair's launch: 8->256 N 4 45^2
-// 61 / 83, 16->128 N 1 20^2 37 / 50, 16->96 N 2 54^2 41 / 55, but 8->256 N 16 32^2
-// 98 / 80.
+// 16 it stays ahead, of more than 96 gradient channels, until the gradient
+// outgrows the pair's launch: 8->256 N 4 45^2 61 / 83, 16->128 N 1 20^2 37 / 50, but
+// 8->256 N 16 32^2 98 / 80. Up to 96 are one and a half of the split weight
+// gradient's 64-row tiles and little work for the input gradient's chain: there
+// the pair gains over a few large images, 16->96 N 2 54^2 41 / 55, and loses over
+// less or over small ones, 8->96 N 2 25^2 47 / 33, N 31 31^2 63 / 46.
 inline bool slab_pair_better(const SlabWgrad& w) {
     const int64_t pixels = (int64_t)w.H * w.W, size = (int64_t)w.C * w.C * w.M * w.N;
     const int taps = w.kh * w.kw;
     if (taps > 9 || w.stride != 1) return false;
     if (taps > 1 && w.M > 64 && w.C > 16 && w.C <= 32 && w.N * pixels <= 16384) return true;
-    if (taps > 1 && w.M > 64 && w.C <= 16 && w.N * pixels * w.M <= 4 << 20) return true;
+    if (taps > 1 && w.M > 64 && w.C <= 16 && w.N * pixels * w.M <= 5 << 19 &&
+        (w.M > 96 || (w.N * pixels > 6144 && pixels >= 1296)))
+        return true;
     if (w.H > 16 || w.W > 16) return false;
     if (pixels <= (w.OW % 4 ? 225 : 196) && size <= (taps == 1 && pixels <= 100 ? 20 : 15) << 20) return true;
     if (w.C * w.M <= 512) return pixels <= 64 || (w.N > 128 && pixels <= 196);
