@@ -114,7 +114,9 @@ inline bool pipe_backward_better(const SlabWgrad& w, bool dinput) {
 // 64x64 and batches of 1 .. 256: the choice is 0.8% from the better one in the
 // mean, and the split tiles alone 4.7%, up to three times: 4->8 1x1 N 208 37^2
 // 14.5 / 44, 1->16 3x3 N 218 63^2 46 / 108, 1->32 N 161 63^2 1x1 53 / 85, but
-// 3->32 3x3 N 32 64^2 121 / 21.
+// 3->32 3x3 N 32 64^2 121 / 21. The direct kernel has to be ahead by more than the
+// fits are usually wrong: of 372 other layers where it was by any margin, 27 were
+// 5 to 40% slower (4->128 1x1 N 205 37^2 120 / 85), by 7% 6.
 inline bool small_wgrad_better(const SlabWgrad& w) {
     const int64_t taps = (int64_t)w.C * w.kh * w.kw, P = (int64_t)w.OH * w.OW;
     if (w.N * w.M * (taps + 1) > INT32_MAX) return false;  // (small_wgrad's partials)
@@ -124,7 +126,8 @@ inline bool small_wgrad_better(const SlabWgrad& w) {
     const double small = base[cls] + round[cls] * groups * (1 + kpx) + image[cls] * kpx;
     const int64_t quads = w.N * w.OH * ((w.OW + 3) / 4);
     const double step = w.OW % 4 ? 1.06 : w.stride == 1 && w.pad <= 1 && w.W >= 4 ? 0.7 : 0.88;
-    return small < 9.2 + step * (double)((w.M + 63) / 64) * (double)quads / (8 * 256);
+    const double split = 9.2 + step * (double)((w.M + 63) / 64) * (double)quads / (8 * 256);
+    return small < 0.93 * split;
 }
 
 // Whether the im2col lowering (three launches) of a weight gradient past the
