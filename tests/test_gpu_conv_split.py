@@ -53,7 +53,9 @@ SHAPES = [  # n, c_in, c_out, h, w, kh, kw, stride, pad
     # ones take, cancel, and its error has no bound element by element)
     (1, 16, 32, 5, 6, 3, 3, 1, 0),
     (1, 9, 70, 1, 4, 3, 3, 1, 1),        # one output row of one quad
-    (3, 256, 160, 7, 7, 3, 3, 1, 1),
+    (3, 256, 160, 7, 7, 3, 3, 1, 1),     # the sum of 6 slices, 8 waves a group
+    (2, 48, 70, 8, 12, 3, 3, 2, 1),      # of 2 slices, two groups a workgroup
+    (3, 48, 70, 8, 12, 3, 3, 2, 1),      # of 3, a wave of four with none
     # layers that the rules leave to the kernels before the split tiles: a weight
     # gradient of few columns, of many over few pixels, and the backward pair
     (30, 4, 8, 21, 23, 1, 1, 1, 0),
